@@ -103,6 +103,10 @@ struct vrestir_handle {
     bool inBatch = false;  // staged by a batch, whose TraceRays step is one kernel
     SplitBufs split{};
     size_t splitPixels = 0;
+    // the open frame's camera-ray profiles: the buffers, and whether they are made (on which stream)
+    DevBuf profTau, profMeta;
+    bool profReady = false;
+    hipStream_t profStream = nullptr;
     // textured environment map: texels, importance mip chain, orientation now and at the last frame
     float* envTexDev = nullptr;
     float* envImpDev = nullptr;
@@ -166,6 +170,11 @@ static void freeLearned(vrestir_handle* h) {
     h->lPartialWaves = 0; h->lCdfPixels = 0; h->lRecSlots = 0;
 }
 
+static void freeProfile(vrestir_handle* h) {
+    freeBuf(h->profTau);
+    freeBuf(h->profMeta);
+    h->profReady = false;
+}
 static void freeSplit(vrestir_handle* h) {
     dfree(h->split.recs); dfree(h->split.trs); dfree(h->split.dens); dfree(h->split.counts); dfree(h->split.plan);
     dfree(h->split.fix);
@@ -355,6 +364,7 @@ extern "C" int32_t vrestir_destroy(vrestir_handle* h) {
     dfree(h->relPartial);
     dfree(h->relOut);
     freeSplit(h);
+    freeProfile(h);
     freeLearned(h);
     delete h;
     return VRESTIR_OK;
@@ -391,6 +401,7 @@ extern "C" int32_t vrestir_frame_count(const vrestir_handle* h, int32_t* out) {
 
 // ------------------------------------------------------------------ scene
 static int uploadScene(vrestir_handle* h) {
+    h->profReady = false;
     HIPCHK(h, hipSetDevice(h->device));
     HIPCHK(h, hipDeviceSynchronize());
     HIPCHK(h, hipMemcpy(h->sceneDev, &h->sceneHost, sizeof(Scene), hipMemcpyHostToDevice));
@@ -1387,6 +1398,7 @@ extern "C" int32_t vrestir_prepare_frame(vrestir_handle* h, int32_t W, int32_t H
         if (rc) return rc;
     }
     h->totalRoundId = 0;
+    h->profReady = false;
     h->frameOpen = true;
     return VRESTIR_OK;
 }
@@ -1498,6 +1510,64 @@ static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
     return VRESTIR_OK;
 }
 
+// The camera-ray profiles of the open frame (profileTr in vr_pass.hpp): made when the
+// spatial visibility rays are ray-marched and the stages run in their split forms.
+// A row has an entry per march step of the longest ray the grid can have (its
+// diagonal); rows that would not fit the budget or three quarters of the free memory
+// are not made, and the rays are traced where they are needed.
+static const size_t kProfileBudget = (size_t)16 << 30;
+static void profilePlan(vrestir_handle* h, Frame& F) {
+    F.prof = CamProfile{};
+    const vrestir_params& p = h->P;
+    const Options& so = F.spatialOpt;
+    if (h->splitReuse != 2 || so.visibilityTrackingMethod != 2u || p.useReference || p.useSurfaceScene || F.noReuse ||
+        h->freezeFrame)
+        return;
+    const Scene& S = h->sceneHost;
+    const int slot = so.visibilityMipLevel;
+    const Grid& G = S.grid[slot];
+    if (!G.valid) return;
+    const double tStep = (double)S.tStep * S.worldScaling * so.visibilityTStepScale * (slot + 1);
+    // world vectors of the box's edges: rows of the inverse of w2i's linear part, times its sizes
+    const float* M = G.w2i;
+    const double m[9] = {M[0], M[1], M[2], M[4], M[5], M[6], M[8], M[9], M[10]};
+    const double det = m[0] * (m[4] * m[8] - m[5] * m[7]) - m[1] * (m[3] * m[8] - m[5] * m[6]) +
+                       m[2] * (m[3] * m[7] - m[4] * m[6]);
+    const double inv[9] = {m[4] * m[8] - m[5] * m[7], m[2] * m[7] - m[1] * m[8], m[1] * m[5] - m[2] * m[4],
+                           m[5] * m[6] - m[3] * m[8], m[0] * m[8] - m[2] * m[6], m[2] * m[3] - m[0] * m[5],
+                           m[3] * m[7] - m[4] * m[6], m[1] * m[6] - m[0] * m[7], m[0] * m[4] - m[1] * m[3]};
+    double longest = 0.0;
+    for (int c = 0; c < 4; c++) {
+        double l2 = 0.0;
+        for (int k = 0; k < 3; k++) {
+            const double e = (G.bmax[0] * inv[k] + (c & 1 ? -1 : 1) * G.bmax[1] * inv[3 + k] +
+                              (c & 2 ? -1 : 1) * G.bmax[2] * inv[6 + k]) / det;
+            l2 += e * e;
+        }
+        longest = std::max(longest, std::sqrt(l2));
+    }
+    const double steps = longest / tStep + 2.0;
+    if (!(steps > 0.0) || !(steps < 65000.0)) return;
+    const size_t n = (size_t)h->W * h->H, rowLen = (size_t)steps + 1;
+    const size_t need = n * rowLen * sizeof(float), meta = n * 2 * sizeof(float);
+    if (need > kProfileBudget) return;
+    if (need > h->profTau.cap) {
+        size_t freeB = 0, totalB = 0;
+        if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || need > (freeB + h->profTau.cap) / 4 * 3) return;
+    }
+    void *tau = nullptr, *mt = nullptr;
+    const void* before = h->profTau.p;
+    if (growBuf(h->profTau, need, &tau) != hipSuccess || growBuf(h->profMeta, meta, &mt) != hipSuccess) {
+        (void)hipGetLastError();
+        freeProfile(h);
+        return;
+    }
+    if (tau != before) h->profReady = false;
+    F.prof.tau = (float*)tau;
+    F.prof.meta = (float*)mt;
+    F.prof.rowLen = (int32_t)rowLen;
+}
+
 // Implementation choices with no counterpart in the reference.
 extern "C" int32_t vrestir_set_tuning(vrestir_handle* h, int32_t key, int32_t value) {
     if (!h) return VRESTIR_EINVAL;
@@ -1509,7 +1579,9 @@ extern "C" int32_t vrestir_set_tuning(vrestir_handle* h, int32_t key, int32_t va
                 HIPCHK(h, hipSetDevice(h->device));
                 HIPCHK(h, hipDeviceSynchronize());
                 freeSplit(h);
+                freeProfile(h);
             }
+            h->profReady = false;
             return VRESTIR_OK;
         case VRESTIR_TUNE_SPLIT_TRACE:
             if (value < 0 || value > 1) return fail(h, VRESTIR_EINVAL, "split TraceRays must be 0 or 1");
@@ -1602,7 +1674,7 @@ static int stageArgs(vrestir_handle* h, hipStream_t st, int stage, int round, fl
     const Frame& F = h->frame;
     int oa = -1, ob = -1;
     switch (stage) {
-        case VRESTIR_STAGE_GENERATE_FEATURES: oa = 0; break;
+        case VRESTIR_STAGE_GENERATE_FEATURES: oa = 0; ob = F.spatialOpt.visibilityMipLevel; break;
         case VRESTIR_STAGE_TRACE_RAYS:
             if (p.useReference) oa = 0;
             else { oa = F.initialOpt.visibilityMipLevel; ob = F.initialOpt.lightingMipLevel; }
@@ -1614,6 +1686,8 @@ static int stageArgs(vrestir_handle* h, hipStream_t st, int stage, int round, fl
         case VRESTIR_STAGE_FINAL_SHADING: oa = F.finalOpt.visibilityMipLevel; ob = 0; break;
         default: break;
     }
+    if (stage != VRESTIR_STAGE_COPY_RESERVOIRS && stage != VRESTIR_STAGE_FINAL_SHADING) profilePlan(h, a.frame);
+    if (stage == VRESTIR_STAGE_GENERATE_FEATURES && !a.frame.prof.tau) ob = -1;
     a.occBytes = occPlan(h, oa, ob, a.frame.occSlot);
     if (stage == VRESTIR_STAGE_TRACE_RAYS || stage == VRESTIR_STAGE_TEMPORAL_REUSE ||
         stage == VRESTIR_STAGE_SPATIAL_REUSE || stage == VRESTIR_STAGE_FINAL_SHADING) {
@@ -1637,6 +1711,13 @@ extern "C" int32_t vrestir_run_stage(vrestir_handle* h, void* stream, int32_t st
     if (rc) return rc;
     const size_t n = (size_t)h->W * h->H, ne = n * (size_t)std::max(p.maxBounces - 1, 1);
     const int t = h->totalRoundId;
+    // the profiles: GenerateFeatures makes them; a stage run without it, or on another
+    // stream than they were made on, makes its own first
+    if (a.frame.prof.tau) {
+        if (stage != VRESTIR_STAGE_GENERATE_FEATURES && (!h->profReady || h->profStream != st)) HIPCHK(h, launchProfile(a));
+        h->profReady = true;
+        h->profStream = st;
+    }
     HIPCHK(h, launchStage(a));
     if (stage == VRESTIR_STAGE_TEMPORAL_REUSE) {
         if (!p.enableSpatialReuse) {
@@ -2031,6 +2112,7 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
     // steps with op < 0 are per-pass launches of the learned stages (-1 proposal, -2 training)
     struct Step { int op, stage, round; };
     std::vector<Step> steps = {{kOpFeatures, VRESTIR_STAGE_GENERATE_FEATURES, 0}};
+    steps.push_back({kOpProfile, VRESTIR_STAGE_GENERATE_FEATURES, 0});
     if (learned) steps.push_back({-1, VRESTIR_STAGE_LEARNED_PROPOSAL, 0});
     steps.push_back({learned ? kOpTraceLearned : kOpTrace, VRESTIR_STAGE_TRACE_RAYS, 0});
     if (learned) steps.push_back({-2, VRESTIR_STAGE_LEARNED_TRAIN, 0});

@@ -5,11 +5,21 @@
 namespace vr {
 
 // GenerateFeatures (VR/GenerateFeatures.cs.slang:57-102); the body is in vr_stages.hpp.
+// The camera-ray profiles need nothing but the camera either: they ride along as a
+// second layer of workgroups (z = 1), so a small frame pays one march's latency.
 __global__ __launch_bounds__(256) void kFeatures(const Scene* __restrict__ sc, const Frame fr,
                                                  float2* __restrict__ features, VItem* __restrict__ vbuf) {
-    featuresBody(sc, fr, features, vbuf, launchBlock());
+    if (blockIdx.z == 0) featuresBody(sc, fr, features, vbuf, launchBlock());
+    else profileBody(sc, fr, launchBlock());
 }
-
+// The profiles alone, for a stage that runs without GenerateFeatures before it.
+__global__ __launch_bounds__(256) void kProfile(const Scene* __restrict__ sc, const Frame fr) {
+    profileBody(sc, fr, launchBlock());
+}
+hipError_t launchProfile(const LaunchArgs& a) {
+    hipLaunchKernelGGL(kProfile, tiles(a.width, a.height), dim3(256), a.occBytes, a.stream, a.scene, a.frame);
+    return hipGetLastError();
+}
 
 // The hierarchical walk's visit sequence: the occupied bricks handed to a
 // tracker, hashed in order (FNV-1a over their index-space minima).
@@ -192,7 +202,10 @@ __global__ __launch_bounds__(256) void kTrack(const Scene* __restrict__ sc, cons
 hipError_t launchStage(const LaunchArgs& a) {
     const dim3 g = tiles(a.width, a.height), blk(256, 1, 1);
     switch (a.stage) {
-        case 0: hipLaunchKernelGGL(kFeatures, g, blk, a.occBytes, a.stream, a.scene, a.frame, a.features, a.vbuf); break;
+        case 0:
+            hipLaunchKernelGGL(kFeatures, dim3(g.x, g.y, a.frame.prof.tau ? 2 : 1), blk, a.occBytes, a.stream, a.scene,
+                               a.frame, a.features, a.vbuf);
+            break;
         case 1: return launchTraceRays(a);
         case 2: return launchTemporalReuse(a);
         case 3: return launchSpatialReuse(a);

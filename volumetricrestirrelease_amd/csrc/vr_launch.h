@@ -41,6 +41,8 @@ struct LaunchArgs {
 };
 
 hipError_t launchStage(const LaunchArgs& a);
+// The frame's camera-ray profiles (frame.prof); GenerateFeatures makes them too.
+hipError_t launchProfile(const LaunchArgs& a);
 // Per-stage launchers, one translation unit each (vr_k_*.hip).
 hipError_t launchTraceRays(const LaunchArgs& a);
 void latticeSize(int width, int height, int stride, int& lw, int& lh);
@@ -71,7 +73,7 @@ struct BatchList {
 enum BatchOp {
     kOpFeatures = 0, kOpTrace, kOpTemporalRecord, kOpTemporalReplay, kOpCopyFeatures, kOpSpatialRecord,
     kOpSpatialReplay, kOpCopyReservoirs, kOpFinalRecord, kOpFinalReplay, kOpSegmentsMarch, kOpSegmentsCells,
-    kOpTraceLearned, kOpTemporalDirect, kOpCount
+    kOpTraceLearned, kOpTemporalDirect, kOpProfile, kOpCount
 };
 // One persistent launch of `grid` workgroups draining the step's work list
 // (counter: the step's queue head, zero before the launch). args and list are

@@ -412,9 +412,75 @@ VR_DEV v3 directLightingPT(const Scene& S, const EnvXf& X, Rng& rng, const Mediu
 // and the replay reads them back in the same order instead of fetching the
 // volume again. An evaluation makes at most b lookups and may record b + 1
 // rays, so a pixel's ray capacity bounds its lookups too.
+// ------------------------------------------------------------------ camera-ray profiles
+// A target evaluation starts with the transmittance of a pixel's camera ray up to
+// the sample's depth, and one frame asks for the same ray at many depths: a pixel's
+// ray serves its own evaluations and those of every neighbour that weighs a sample
+// against it (K (K - 1) evaluations per pixel and spatial round). The ray-marched
+// samples of a ray do not depend on where it ends: a shorter ray takes the same
+// samples, those before its end. So each ray is marched once per frame
+// (ProfileMarch, the full ray) and its running optical depth kept per march step;
+// a query is then one lookup instead of a walk. At 1080p on a 512^3 cloud (path
+// length 3, 2 rounds of 5 neighbours) the frame's segment traces go from 31.0 to
+// 17.2 ms; making the rows adds 0.44 ms to GenerateFeatures' launch, the lookups
+// 0.14 ms to each spatial record.
+//
+// Step k of a ray covers [tNear + k tStep, tNear + (k + 1) tStep) and holds at most
+// one sample, at its centre (the trackers snap every brick's first sample to that
+// grid). Entry e of a row is the optical depth of the samples of steps <= k0 + e.
+// Where the walk of a ray that ends at `depth` could take other samples, the
+// lookup declines and the ray is traced as before:
+//   * a depth within rounding of a step's centre;
+//   * NaN entries, written for samples in the first brick of a 128^3 block that
+//     lie before the brick's tx = entry + 0.01: the hierarchical walk leaves a ray
+//     out of that brick when its end lies between the sample and tx;
+//   * a ray longer than the row (kProfileNone).
+// pixel < 0: not one of this frame's camera rays.
+VR_DEV bool profileTr(const Scene& S, const CamProfile& P, const Options& o, int pixel, float depth, float& Tr) {
+    if (!P.tau || pixel < 0) return false;
+    const float2 m = reinterpret_cast<const float2*>(P.meta)[pixel];
+    const uint32_t w = __float_as_uint(m.y);
+    const int k0 = (int)(w & 0xFFFFu), len = (int)(w >> 16);
+    if (w == kProfileNone) return false;
+    Tr = 1.f;
+    if (len == 0) return true;
+    const int slot = o.visibilityMipLevel;
+    const float tStep = S.tStep * S.worldScaling * o.visibilityTStepScale * (float)((slot >= 8 ? slot - 8 : slot) + 1);
+    // step k's sample counts when its centre lies before depth: k < x. t is rounded at
+    // each of a brick's up to 128 steps, so within tol of a centre either may hold
+    const float inv = 1.f / tStep;
+    const float x = (depth - m.x) * inv - 0.5f;
+    const float tol = 1e-5f * (fabsf(m.x) * inv + (float)(k0 + len));
+    if (!(tol < 0.25f) || isnan(x)) return false;
+    if (x < (float)k0 - 0.5f) return true;
+    int e = len - 1;
+    if (x < (float)(k0 + len) - 0.5f) {
+        if (fabsf(x - rintf(x)) <= tol) return false;
+        e = (int)ceilf(x) - 1 - k0;
+    }
+    if (e < 0) return true;
+    const float tau = P.tau[(size_t)pixel * P.rowLen + e];
+    if (isnan(tau)) return false;
+    Tr = expf(-tau);
+    return true;
+}
+
 template <int VM, int LM>
 struct DirectTrace {
     static constexpr bool kSplit = false;
+    const CamProfile* prof = nullptr;
+    // vis of kind 0 for pixel's camera ray
+    VR_DEV float camVis(const Scene& S, const Ray& r, Rng& rng, const Options& o, bool isFinal, int off, int pixel) {
+        if constexpr (VM == 2) {
+            float Tr;
+            if (prof && !isFinal && off == 0 && profileTr(S, *prof, o, pixel, r.tMax, Tr)) {
+                float v = 0.f;
+                for (int i = 0; i < o.visibilitySamples; i++) v += Tr;
+                return v / (float)o.visibilitySamples;
+            }
+        }
+        return vis(S, r, rng, o, 0, isFinal, off);
+    }
     // kind 0: visibility options; 1: lighting options (grid 0 in final shading).
     // off: kPrevDensityOffset for the previous frame's grids, else 0.
     VR_DEV float vis(const Scene& S, const Ray& r, Rng& rng, const Options& o, int kind, bool isFinal, int off) {
@@ -454,6 +520,16 @@ struct RecordTrace {
         dens[(size_t)nd++ * dstride] = d;
         return d;
     }
+    // A camera ray's transmittance from its profile goes to the density slots (with
+    // at most b lookups an evaluation's b + 1 slots hold it too); -1 there: recorded.
+    const CamProfile* prof = nullptr;
+    VR_DEV float camVis(const Scene& S, const Ray& r, Rng& rng, const Options& o, bool isFinal, int off, int pixel) {
+        if (!prof || !prof->tau || isFinal || o.visibilitySamples <= 0) return vis(S, r, rng, o, 0, isFinal, off);
+        float Tr;
+        const bool known = off == 0 && profileTr(S, *prof, o, pixel, r.tMax, Tr);
+        dens[(size_t)nd++ * dstride] = known ? Tr : -1.f;
+        return known ? sameSamples(1.f, o.visibilitySamples) : vis(S, r, rng, o, 0, isFinal, off);
+    }
 };
 struct ReplayTrace {
     static constexpr bool kSplit = true;
@@ -469,6 +545,12 @@ struct ReplayTrace {
     size_t dstride;
     int nd;
     VR_DEV float density(const Scene&, int, v3) { return dens[(size_t)nd++ * dstride]; }
+    const CamProfile* prof = nullptr;
+    VR_DEV float camVis(const Scene& S, const Ray& r, Rng& rng, const Options& o, bool isFinal, int off, int) {
+        if (!prof || !prof->tau || isFinal || o.visibilitySamples <= 0) return vis(S, r, rng, o, 0, isFinal, off);
+        const float Tr = dens[(size_t)nd++ * dstride];
+        return Tr >= 0.f ? sameSamples(Tr, o.visibilitySamples) : vis(S, r, rng, o, 0, isFinal, off);
+    }
 };
 
 // SampleDirectLighting (VR/VolumeUtils.slang:454-492); the shadow ray's
@@ -577,7 +659,7 @@ struct CandReplay : ReplayTrace {
 // frame's grids (useLastFrameGrid, VR/ReSTIRHelper.slang:95-96), else 0.
 template <int B, class TP>
 VR_DEV v3 evaluateF(const Scene& S, const EnvXf& X, Res tap, const float* extra, Ray ray, Rng& rng, const Options& opt,
-                    bool noReuse, bool isFinal, TP& tp, int gridOff = 0) {
+                    bool noReuse, bool isFinal, TP& tp, int camPixel, int gridOff = 0) {
     bool isBg = tap.depth == kTMax;
     ray.tMax = tap.depth;
     v3 F = V3(1.f), Fn = V3(1.f);
@@ -590,7 +672,7 @@ VR_DEV v3 evaluateF(const Scene& S, const EnvXf& X, Res tap, const float* extra,
     {
         float density = (isBg || noReuse) ? 1.f : tp.density(S, gridOff, pW);
         if (density == 0.f) return V3(0.f);
-        if (!noReuse) vis = tp.vis(S, ray, rng, opt, 0, isFinal, gridOff);
+        if (!noReuse) vis = tp.camVis(S, ray, rng, opt, isFinal, gridOff, camPixel);
         v3 ss = isBg ? V3(1.f) : (isSelfEmission ? ld3(S.sigma_a) : ld3(S.sigma_s));
         if (noReuse && !isBg) ss = ss / S.sigma_t;
         F = F * (V3(vis * density) * ss);
@@ -692,9 +774,10 @@ VR_DEV v3 evaluateF(const Scene& S, const EnvXf& X, Res tap, const float* extra,
 // The direct form: traces every transmittance ray where evaluateF needs it.
 template <int B, int VM, int LM>
 VR_DEV v3 evaluateF(const Scene& S, const EnvXf& X, const Res& tap, const float* extra, const Ray& ray, Rng& rng,
-                    const Options& opt, bool noReuse, bool isFinal, int gridOff = 0) {
+                    const Options& opt, bool noReuse, bool isFinal, const CamProfile& prof, int camPixel) {
     DirectTrace<VM, LM> tp;
-    return evaluateF<B>(S, X, tap, extra, ray, rng, opt, noReuse, isFinal, tp, gridOff);
+    tp.prof = &prof;
+    return evaluateF<B>(S, X, tap, extra, ray, rng, opt, noReuse, isFinal, tp, camPixel);
 }
 
 // ComputeInitialSample (VR/ComputeInitialSample.slang:4-395). ex[] receives the

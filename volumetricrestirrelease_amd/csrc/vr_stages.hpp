@@ -81,6 +81,66 @@ VR_DEV void featuresBody(const Scene* __restrict__ sc, const Frame& fr, float2* 
     features[px.id] = make_float2(__int_as_float(noSurface), accT);
 }
 
+// TrMarch over a whole camera ray, keeping the running optical depth per march step
+// (the row that profileTr reads).
+struct ProfileMarch {
+    const Scene* S; const Grid* G; bool linear; float tStep; float* row; int rowLen;
+    float Tr = 0.f; float tNear = 0, tFar = 0; Ray ray;
+    int k0 = 0, n = 0, block = -1;  // first step, entries written, the last brick's block
+    bool bad = false;
+    VR_DEV void setRayInfo(float a, float b, const Ray& r) { tNear = a; tFar = b; ray = r; }
+    VR_DEV void start() {}
+    VR_DEV void put(int k, float v, float before) {
+        if (n == 0) k0 = k;
+        const int e = k - k0;
+        if (e < n || e >= rowLen || k > 0xFFFF || e >= 0xFFFF - 1) { bad = true; return; }
+        while (n < e) row[n++] = before;  // steps without a sample
+        row[n++] = v;
+    }
+    VR_DEV bool brickStep(const Dda& dda, const BrickCtx& bc, int, float& t, Rng&) {
+        const int b = ((int)bc.vmin.x >> 7) | ((int)bc.vmin.y >> 7) << 8 | ((int)bc.vmin.z >> 7) << 16;
+        const bool firstOfBlock = b != block;
+        block = b;
+        const float kf = floorf((t - tNear) / tStep);
+        int k = (int)kf;
+        t = tNear + (kf + 0.5f) * tStep;
+        if (t < dda.tx) { t += tStep; k++; }
+        v3 q = at(ray, t) - bc.vmin;
+        const v3 dq = 1.f * tStep * ray.d;
+        for (int iter = 0; iter < 128 && inBrick(q); iter++) {
+            if (t >= tFar) return true;
+            const float before = -Tr;
+            const float st = brickDensity(*S, *G, bc, q, linear) * S->sigma_t;
+            Tr += -st * 1.f * tStep;
+            put(k++, firstOfBlock && t < dda.tx ? __uint_as_float(0x7FC00000u) : -Tr, before);
+            if (bad) return true;
+            q = q + dq;
+            t += 1.f * tStep;
+        }
+        return false;
+    }
+    VR_DEV void end() {}
+};
+// A pixel's camera-ray profile through the grid of the spatial visibility options.
+VR_DEV void profileBody(const Scene* __restrict__ sc, const Frame& fr, VBlock vb) {
+    const Scene& S = *sc;
+    const Frame& F = fr;
+    occCacheLoad(S, F.occSlot[0], F.occSlot[1]);
+    PixelIdx px = pixelOf(F, vb);
+    if (!px.ok) return;
+    Rng rng{0, 0, 0, 0};
+    const Ray r{ld3(F.cam.pos), rayDir(F.cam, px.x, px.y, F.width, F.height), 0.f, kTMax};
+    const int slot = F.spatialOpt.visibilityMipLevel;
+    ProfileMarch a;
+    a.S = &S; a.G = &S.grid[slot]; a.linear = F.spatialOpt.visibilityUseLinearSampler != 0;
+    a.tStep = S.tStep * S.worldScaling * F.spatialOpt.visibilityTStepScale * (float)((slot >= 8 ? slot - 8 : slot) + 1);
+    a.row = F.prof.tau + (size_t)px.id * F.prof.rowLen;
+    a.rowLen = F.prof.rowLen;
+    traverse(S, r, slot, rng, a, false);
+    reinterpret_cast<float2*>(F.prof.meta)[px.id] =
+        make_float2(a.tNear, __uint_as_float(a.bad ? kProfileNone : (uint32_t)a.k0 | (uint32_t)a.n << 16));
+}
+
 // IntegrateByVolumePathTracing (VR/VolumePathTracingFunctions.slang:3-132), NEE on.
 VR_DEV v3 pathTrace(const Scene& S, const Frame& Fr, Ray ray, Rng& rng, int lightSamples, int maxBounces) {
     MediumInteraction mi{V3(0.f), V3(0.f), S.g, false};
@@ -282,7 +342,7 @@ VR_DEV void tracePixel(const Scene& S, const Frame& F, PixelIdx px, ResStore* __
             }
     }
     fin.exStart = exStart;
-    float ph = lum(evaluateF<B, VM, LM>(S, F.env[0], fin, outExtra, ray, rng, F.spatialOpt, false, false));
+    float ph = lum(evaluateF<B, VM, LM>(S, F.env[0], fin, outExtra, ray, rng, F.spatialOpt, false, false, F.prof, px.id));
     if (fin.runningSum > 0.f) {
         fin.runningSum *= fin.p_y == 0.f ? 0.f : ph / fin.p_y;
         fin.p_y = ph;
@@ -356,6 +416,7 @@ VR_DEV void temporalBody(const Scene* __restrict__ sc, const Frame& fr, ResStore
     PixelIdx px = pixelOf(F, vb);
     if (!px.ok) return;
     TracePolicy<MODE, VM, LM> tp;
+    tp.prof = &F.prof;
     if constexpr (MODE == kRecord) { tp.out = sb.recs + (size_t)px.id * sb.cap; tp.n = 0; tp.dens = sb.dens + px.id; tp.dstride = (size_t)F.width * F.height; tp.nd = 0; sb.counts[px.id] = 0; }
     if constexpr (MODE == kReplay) { tp.tr = sb.trs + px.id; tp.trStride = (size_t)F.width * F.height; tp.n = 0; tp.dens = sb.dens + px.id; tp.dstride = (size_t)F.width * F.height; tp.nd = 0; }
     constexpr bool kWrites = MODE != kRecord;
@@ -446,7 +507,7 @@ VR_DEV void temporalBody(const Scene* __restrict__ sc, const Frame& fr, ResStore
             nPy = ti.p_y;
             if (isnan(ti.runningSum) || isinf(ti.runningSum)) ti.runningSum = 0.f;
             if (i > 0 && ti.runningSum != 0.f) {
-                float ph = lum(evaluateF<B>(S, F.env[0], ti, temporalExtra, ray, rng, F.spatialOpt, false, false, tp));
+                float ph = lum(evaluateF<B>(S, F.env[0], ti, temporalExtra, ray, rng, F.spatialOpt, false, false, tp, px.id));
                 float w = ph / ti.p_y;
                 if (isinf(w) || isnan(w)) w = 0.f;
                 ti.runningSum *= w;
@@ -475,7 +536,7 @@ VR_DEV void temporalBody(const Scene* __restrict__ sc, const Frame& fr, ResStore
                     tmp.depth = centerPrevDepth;
                     // isLastFrame (VR/TemporalReuse.cs.slang:335-338): previous orientation and grids
                     float py = lum(evaluateF<B>(S, F.env[1], tmp, curExtra, nr, rng, F.spatialOpt, false, false, tp,
-                                                F.prevGridOffset));
+                                                -1, F.prevGridOffset));
                     if (isinf(py) || isnan(py)) py = 0.f;
                     psum += py * cM;
                 }
@@ -541,6 +602,7 @@ VR_DEV void spatialBody(const Scene* __restrict__ sc, const Frame& fr, int round
     const int K = F.spatialSampleCount;
     const bool talbot = F.spatialMIS == 1;
     TracePolicy<MODE, VM, LM> tp;
+    tp.prof = &F.prof;
     if constexpr (MODE == kRecord) { tp.out = sb.recs + (size_t)px.id * sb.cap; tp.n = 0; tp.dens = sb.dens + px.id; tp.dstride = (size_t)F.width * F.height; tp.nd = 0; }
     if constexpr (MODE == kReplay) { tp.tr = sb.trs + px.id; tp.trStride = (size_t)F.width * F.height; tp.n = 0; tp.dens = sb.dens + px.id; tp.dstride = (size_t)F.width * F.height; tp.nd = 0; }
     uint32_t plan = 0;
@@ -578,7 +640,7 @@ VR_DEV void spatialBody(const Scene* __restrict__ sc, const Frame& fr, int round
         Res tap = loadRes(in, ty * W + tx, B);
         float misW = 1.f;
         if (s > 0 && tap.runningSum != 0.f) {
-            float ph = lum(evaluateF<B>(S, F.env[0], tap, inExtra, ray, rng, F.spatialOpt, false, false, tp));
+            float ph = lum(evaluateF<B>(S, F.env[0], tap, inExtra, ray, rng, F.spatialOpt, false, false, tp, px.id));
             float w = ph / tap.p_y;
             if (isinf(w) || isnan(w)) w = 0.f;
             tap.runningSum *= w;
@@ -605,7 +667,7 @@ VR_DEV void spatialBody(const Scene* __restrict__ sc, const Frame& fr, int round
                     psum += py2 * m2;
                 } else {
                     Ray nr{ray.o, rayDir(F.cam, t2x, t2y, W, H), 0.f, tap.depth};
-                    float py = lum(evaluateF<B>(S, F.env[0], tap, inExtra, nr, rng, F.spatialOpt, false, false, tp));
+                    float py = lum(evaluateF<B>(S, F.env[0], tap, inExtra, nr, rng, F.spatialOpt, false, false, tp, t2));
                     if (isinf(py) || isnan(py)) py = 0.f;
                     psum += py * m2;
                 }
@@ -695,7 +757,7 @@ VR_DEV void finalBody(const Scene* __restrict__ sc, const Frame& fr, const ResSt
         Res r = loadRes(cur, px.id, B);
         if (r.runningSum > 0.f) {
             Ray ray{ld3(F.cam.pos), rayDir(F.cam, px.x, px.y, F.width, F.height), 0.f, r.depth};
-            v3 f = evaluateF<B>(S, F.env[0], r, curExtra, ray, rng, F.finalOpt, F.noReuse != 0, true, tp);
+            v3 f = evaluateF<B>(S, F.env[0], r, curExtra, ray, rng, F.finalOpt, F.noReuse != 0, true, tp, -1);
             float Wt = r.p_y == 0.0f ? 1.f : r.runningSum / (r.p_y * r.M);
             c = c + f * Wt;
         }

@@ -147,6 +147,19 @@ struct CameraFrame {
     float pos[3], U[3], V[3], W[3];
 };
 
+// Optical depths along every pixel's camera ray through the grid of the spatial
+// visibility options (see profileTr in vr_pass.hpp): pixel p's row is
+// tau[p * rowLen ...], meta[p] = {tNear, first step index | row entries << 16}.
+// tau == nullptr: no profile, every camera ray is traced where it is needed.
+struct CamProfile {
+    float* tau;
+    float* meta;                  // 2 floats per pixel
+    int32_t rowLen;
+    int32_t pad_;
+};
+// meta's second word for a row that does not hold its ray (longer than rowLen)
+static const uint32_t kProfileNone = 0xFFFF0000u;
+
 // Per-frame constants (VR/VolumetricReSTIR.cpp:453-496 and the kernels' cbuffers),
 // passed by value as a kernel argument.
 struct Frame {
@@ -180,6 +193,7 @@ struct Frame {
     int32_t hasAnimation;         // the volume advanced a frame of its sequence since the last frame
     int32_t prevGridOffset;       // kPrevDensityOffset when previous-frame grids serve isLastFrame lookups, else 0
     Options initialOpt, spatialOpt, finalOpt;
+    CamProfile prof;
 };
 // A transmittance ray recorded by the record pass of a reuse kernel
 // (world-space origin and direction, tMax, and which options trace it:
