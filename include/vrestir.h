@@ -212,7 +212,7 @@ int32_t vrestir_set_volume(vrestir_handle* h, const vrestir_volume_desc* desc);
  * a ring of two frames and binds it with the frame before it as the previous frame
  * (as vrestir_set_volume_frame(h, i, 1) does for a resident sequence). Later frames
  * keep the first frame's material and need its dimensions, mips, format and grids.
- * Synchronises the device; temporary device memory is about three dense grids. */
+ * Synchronises the device; temporary device memory is about a third of a dense grid. */
 int32_t vrestir_stream_volume_frame(vrestir_handle* h, void* stream, const vrestir_volume_desc* desc);
 /* Binds owner's volume into h read-only (no counterpart in the reference, where the
  * passes of a frame share the Scene): the current and previous frame's grids, the

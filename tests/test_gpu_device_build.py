@@ -195,3 +195,50 @@ def test_shared_volume_renders_like_an_own_copy():
         assert np.array_equal(ia[f], ib[f]), f
     with pytest.raises(VolumetricReSTIRError, match="another handle"):
         shared.addVolumeFrame(specs[1])
+
+
+@pytest.mark.parametrize("dims,mips,fp16,offset", [
+    ((8, 8, 8), 1, False, 0), ((24, 40, 56), 1, True, 1), ((80, 16, 48), 2, False, 3), ((160, 32, 96), 3, True, 0),
+    ((64, 64, 192), 4, False, 2), ((128, 256, 128), 5, True, 0)])
+def test_device_build_at_tile_edges_equals_host_build(dims, mips, fp16, offset):
+    """Grids whose sides leave remainders of the build's 64 x 8 x 8 tiles, every number of
+    levels on both sides of those the tile pass reduces, a source that is not 16-byte
+    aligned (offset floats into an allocation), voxels at the faces, negative values and
+    values below the stored clamp. The residual-ratio tracker reads the bricks' bounds."""
+    import torch
+    nx, ny, nz = dims
+    say(f"case: {nx}x{ny}x{nz}, {mips} mips, {'fp16' if fp16 else 'fp32'}, source offset {offset}")
+    rng = np.random.default_rng(nx + mips)
+    d = rng.uniform(-0.2, 1.0, size=(nz, ny, nx)).astype(np.float32)
+    d[rng.uniform(size=d.shape) < 0.4] = 0.0
+    d[nz // 3: nz // 2] = 0.0
+    d[:, :, nx // 2: nx // 2 + 9] *= (rng.uniform(size=(nz, ny, d[:, :, nx // 2: nx // 2 + 9].shape[2])) < 0.02)
+    d.reshape(-1)[::97] *= 1e-10
+    spec = small_scene(res=8, width=16, height=8)
+    spec.density, spec.num_mips = d, mips
+    spec.brick_format = abi.BRICK_FP16 if fp16 else abi.BRICK_FP32
+    m = np.zeros(16, np.float32)
+    m[0], m[5], m[10], m[15] = 2.0 / nx, 2.0 / ny, 2.0 / nz, 1.0
+    m[12:15] = -1.0
+    spec.index_to_world = m
+    top = mips - 1
+    spec.params.update(initialBaseMipLevel=min(1, top), initialLightingMipLevel=min(2, top),
+                       temporalReprojectionMipLevel=min(1, top), spatialVisibilityMipLevel=min(1, top),
+                       spatialLightingMipLevel=min(1, top))
+    a = VolumetricReSTIR()
+    a.setScene(spec)
+    buf = torch.zeros(d.size + 4, device="cuda")
+    buf[offset: offset + d.size] = dev(d).reshape(-1)
+    b = VolumetricReSTIR()
+    b.setSceneStreamed(spec, buf[offset: offset + d.size])
+    slots = list(range(mips)) + [8 + k for k in range(mips)]
+    same_grids(a, b, slots, rng, n=4096)
+    rays = np.zeros((4096, 8), np.float32)
+    rays[:, :3] = rng.uniform(-1.5, 1.5, size=(4096, 3))
+    dirs = rng.normal(size=(4096, 3))
+    rays[:, 3:6] = dirs / np.linalg.norm(dirs, axis=1, keepdims=True)
+    rays[:, 6] = 3.4e38
+    for slot in slots:
+        ta = track(a, abi.TRACK_TR_RESIDUAL_RATIO, slot, 1, rays)
+        tb = track(b, abi.TRACK_TR_RESIDUAL_RATIO, slot, 1, rays)
+        assert np.array_equal(ta.view(np.uint32), tb.view(np.uint32)), slot

@@ -556,7 +556,6 @@ static int buildFrameDevice(vrestir_handle* h, hipStream_t st, const vrestir_vol
         f.meta[s] = HostGrid();
     }
     const bool fp16 = d.brickFormat == VRESTIR_BRICK_FP16;
-    const size_t n = (size_t)d.nx * d.ny * d.nz;
     auto tmp = [&](int key, size_t bytes, void** p) -> int {
         HIPCHK(h, growBuf(h->buildTmp[key], bytes, p));
         return VRESTIR_OK;
@@ -566,66 +565,109 @@ static int buildFrameDevice(vrestir_handle* h, hipStream_t st, const vrestir_vol
         if (r) freeFrame(f);
         return r;
     };
-    float *cur = nullptr, *cons = nullptr;
-    // per-build counters: [0] and [19] non-finite density / temperature values; the
-    // largest value of each grid as float bits: mip k at [1 + k], conservative mip k
-    // at [9 + k], temperature at [17] (each left by the kernel that writes the grid)
-    unsigned* stats = nullptr;
-    void* scratch = nullptr;
-    if ((rc = tmp(0, n * 4, (void**)&cur)) || (rc = tmp(1, n * 4, (void**)&cons)) ||
-        (rc = tmp(17, 20 * sizeof(unsigned), (void**)&stats)) ||
-        (rc = tmp(18, buildScratchBytes(d.nx, d.ny, d.nz), &scratch)))
-        return done(rc);
-    HIPCHK(h, hipMemsetAsync(stats, 0, 20 * sizeof(unsigned), st));
-    // values are clamped to >= 0; a non-finite one is refused, as the host build refuses it
-    auto clampChecked = [&](const float* src, float* dst, int badAt, int maxAt, const char* what) -> int {
-        int nbad = 0;
-        HIPCHK(h, buildClamp(st, src, dst, n, (int*)stats + badAt, stats + maxAt));
-        HIPCHK(h, hipMemcpyAsync(&nbad, stats + badAt, 4, hipMemcpyDeviceToHost, st));
-        HIPCHK(h, hipStreamSynchronize(st));
-        if (nbad) return fail(h, VRESTIR_EINVAL, std::string("the ") + what + " grid holds a non-finite value");
-        return VRESTIR_OK;
+    // the slots: mip k and its conservative twin, the temperature grid
+    struct Slot { int id, scale; };
+    std::vector<Slot> slots;
+    std::vector<BuildGrid> grids;
+    size_t cells = 0;
+    auto add = [&](int id, int level, const float* src, bool dilate) {
+        BuildGrid g{};
+        g.src = src;
+        g.nx = d.nx >> level; g.ny = d.ny >> level; g.nz = d.nz >> level;
+        g.nnx = (g.nx + 127) / 128; g.nny = (g.ny + 127) / 128; g.nnz = (g.nz + 127) / 128;
+        g.cells = (size_t)(g.nx / 8) * (g.ny / 8) * (g.nz / 8);
+        g.blocks = (size_t)g.nnx * g.nny * g.nnz;
+        g.dilate = dilate;
+        cells += (g.cells + 63) / 64 * 64;
+        slots.push_back({id, 1 << level});
+        grids.push_back(g);
     };
-    auto slot = [&](int s, const float* g, int nx, int ny, int nz, int scale, int maxAt) -> int {
-        uint32_t nb = 0;
-        float mv = 0.f;
-        const BuildAlloc alloc = [&f, s](int kind, size_t bytes, void** p) { return growBuf(f.built[s][kind], bytes, p); };
-        HIPCHK(h, buildSlotDevice(st, g, nx, ny, nz, stats + maxAt, fp16, scratch, f.grids[s], nb, mv, alloc));
-        mipTransform(d.indexToWorld, scale, f.grids[s].w2i);
-        HostGrid& m = f.meta[s];
-        m = HostGrid();
-        m.valid = true; m.nx = nx; m.ny = ny; m.nz = nz; m.numBricks = nb; m.maxValue = mv; m.fp16 = fp16;
-        m.channels = 1; m.nbx = nx / 8; m.nby = ny / 8; m.nbz = nz / 8;
-        m.nnx = f.grids[s].nnx; m.nny = f.grids[s].nny; m.nnz = f.grids[s].nnz;
-        return VRESTIR_OK;
-    };
-    // a failed launch leaves through done(), which releases the temporaries
+    // level k's grids (k > 0) are the handle's temporaries; level 0 is read from the caller's grid
+    for (int k = 0; k < d.numMips; k++) {
+        const size_t m = ((size_t)d.nx >> k) * ((size_t)d.ny >> k) * ((size_t)d.nz >> k);
+        float *n2 = nullptr, *c2 = nullptr;
+        if (k > 0 && ((rc = tmp(2 * k, m * 4, (void**)&n2)) || (rc = tmp(2 * k + 1, m * 4, (void**)&c2)))) return done(rc);
+        add(k, k, k ? n2 : d.density, false);
+        add(8 + k, k, k ? c2 : d.density, k == 0);
+    }
+    if (d.temperature) add(kTemperatureSlot, 0, d.temperature, false);
+    const int ns = (int)grids.size();
+    // scratch: the statistics, then every slot's brick maxima and brick cells
+    const size_t statWords = (sizeof(BuildStats) + 255) / 256 * 64;
+    char* scratch = nullptr;
+    if ((rc = tmp(18, (statWords + 2 * cells) * 4, (void**)&scratch))) return done(rc);
+    BuildStats* stats = (BuildStats*)scratch;
+    unsigned* at = (unsigned*)scratch + statWords;
+    for (BuildGrid& g : grids) { g.brickMax = at; at += (g.cells + 63) / 64 * 64; }
+    for (BuildGrid& g : grids) { g.cellOf = at; at += (g.cells + 63) / 64 * 64; }
+    // a failed launch leaves through done(), which releases the frame's buffers
     auto ck = [&](hipError_t e, const char* what) -> int {
         return e == hipSuccess ? VRESTIR_OK : fail(h, VRESTIR_EHIP, std::string(what) + ": " + hipGetErrorString(e));
     };
-    if ((rc = clampChecked(d.density, cur, 0, 1, "density"))) return done(rc);
-    if ((rc = ck(buildDilate(st, cur, cons, d.nx, d.ny, d.nz, stats + 9), "buildDilate"))) return done(rc);
-    int nx = d.nx, ny = d.ny, nz = d.nz;
-    for (int k = 0; k < d.numMips; k++) {
-        if (k > 0) {
-            float *n2 = nullptr, *c2 = nullptr;
-            const size_t m = (size_t)(nx / 2) * (ny / 2) * (nz / 2);
-            if ((rc = tmp(2 * k, m * 4, (void**)&n2)) || (rc = tmp(2 * k + 1, m * 4, (void**)&c2))) return done(rc);
-            if ((rc = ck(buildReduce2(st, cur, n2, nx, ny, nz, stats + 1 + k), "buildReduce2")) ||
-                (rc = ck(buildReduce2(st, cons, c2, nx, ny, nz, stats + 9 + k), "buildReduce2")))
-                return done(rc);
-            cur = n2; cons = c2;
-            nx /= 2; ny /= 2; nz /= 2;
-        }
-        if ((rc = slot(k, cur, nx, ny, nz, 1 << k, 1 + k)) || (rc = slot(8 + k, cons, nx, ny, nz, 1 << k, 9 + k)))
+    for (int i = 0; i < ns; i++) {
+        BuildGrid& g = grids[i];
+        DevBuf* b = f.built[slots[i].id];
+        if ((rc = ck(growBuf(b[kBufTable], g.cells * 4, (void**)&g.table), "brick table")) ||
+            (rc = ck(growBuf(b[kBufNodes], g.blocks * 4, (void**)&g.nodes), "block table")) ||
+            (rc = ck(growBuf(b[kBufWords], (g.cells + 31) / 32 * 8, (void**)&g.words), "occupancy words")))
             return done(rc);
     }
-    if (d.temperature) {
-        // one full-resolution slot with mip 0's transform
-        float* t = nullptr;
-        if ((rc = tmp(16, n * 4, (void**)&t))) return done(rc);
-        if ((rc = clampChecked(d.temperature, t, 19, 17, "temperature"))) return done(rc);
-        if ((rc = slot(kTemperatureSlot, t, d.nx, d.ny, d.nz, 1, 17))) return done(rc);
+    const int levels = std::min(d.numMips, 4) - 1;
+    float* out[2][4] = {};
+    unsigned* bmax[2][4] = {};
+    for (int l = 0; l <= levels; l++)
+        for (int c = 0; c < 2; c++) {
+            out[c][l] = l ? const_cast<float*>(grids[2 * l + c].src) : nullptr;
+            bmax[c][l] = grids[2 * l + c].brickMax;
+        }
+    if ((rc = ck(buildClear(st, scratch, statWords + cells), "buildClear")) ||
+        (rc = ck(buildLevels(st, d.density, d.nx, d.ny, d.nz, levels, out, bmax, stats->bad), "buildLevels")))
+        return done(rc);
+    for (int k = 4; k < d.numMips; k++)
+        for (int c = 0; c < 2; c++) {
+            const BuildGrid &s = grids[2 * (k - 1) + c], &g = grids[2 * k + c];
+            if ((rc = ck(buildReduce2(st, s.src, const_cast<float*>(g.src), s.nx, s.ny, s.nz), "buildReduce2")) ||
+                (rc = ck(buildBrickMax(st, g.src, g.nx, g.ny, g.nz, g.brickMax, stats->bad), "buildBrickMax")))
+                return done(rc);
+        }
+    if (d.temperature)
+        if ((rc = ck(buildBrickMax(st, d.temperature, d.nx, d.ny, d.nz, grids[ns - 1].brickMax, stats->bad + 1),
+                     "buildBrickMax")))
+            return done(rc);
+    if ((rc = ck(buildTables(st, grids.data(), ns, fp16, stats), "buildTables"))) return done(rc);
+    // the one wait of the build: the brick counts size the pools
+    BuildStats got;
+    if ((rc = ck(hipMemcpyAsync(&got, stats, sizeof(got), hipMemcpyDeviceToHost, st), "build statistics")) ||
+        (rc = ck(hipStreamSynchronize(st), "build statistics")))
+        return done(rc);
+    // a non-finite value is refused, as the host build refuses it
+    for (int k = 0; k < 2; k++)
+        if (got.bad[k])
+            return done(fail(h, VRESTIR_EINVAL, std::string("the ") + (k ? "temperature" : "density") +
+                                                    " grid holds a non-finite value"));
+    for (int i = 0; i < ns; i++) {
+        BuildGrid& g = grids[i];
+        DevBuf* b = f.built[slots[i].id];
+        // an animation's brick counts drift: an eighth more than needed, so few frames reallocate
+        auto grow = [](DevBuf& db, size_t bytes, void** p) {
+            return growBuf(db, db.cap < bytes && db.cap ? bytes + bytes / 8 : bytes, p);
+        };
+        const size_t nb = got.count[i];
+        if ((rc = ck(grow(b[kBufBounds], nb * 16, (void**)&g.bounds), "brick bounds")) ||
+            (rc = ck(grow(b[kBufPool], nb * kBrickVals * (fp16 ? 2 : 4), &g.pool), "brick pool")))
+            return done(rc);
+    }
+    if ((rc = ck(buildFill(st, grids.data(), got, ns, fp16), "buildFill"))) return done(rc);
+    for (int i = 0; i < ns; i++) {
+        const BuildGrid& g = grids[i];
+        Grid& G = f.grids[slots[i].id];
+        buildDescribe(g, got, i, fp16, G);
+        mipTransform(d.indexToWorld, slots[i].scale, G.w2i);
+        HostGrid& m = f.meta[slots[i].id];
+        m = HostGrid();
+        m.valid = true; m.nx = g.nx; m.ny = g.ny; m.nz = g.nz; m.numBricks = got.count[i]; m.maxValue = G.maxValue;
+        m.fp16 = fp16; m.channels = 1; m.nbx = G.nbx; m.nby = G.nby; m.nbz = G.nbz;
+        m.nnx = g.nnx; m.nny = g.nny; m.nnz = g.nnz;
     }
     HostVolume hv;
     volumeSpacing(d.indexToWorld, hv);

@@ -9,11 +9,22 @@
 // grid, the tiny-value clamp against the grid maximum, round-to-nearest-even
 // fp16, and a brick's bounds summed over its 10^3 apron with x outermost), so a
 // device-built slot equals the host-built slot byte for byte.
+//
+// HBM bounds a large build, launches and waits a small one. The dense grid is read
+// once for everything that is not a brick (kLevels: both mip chains and the largest
+// value of every brick of every level), the full-resolution clamped and dilated
+// grids are never stored (the fills of their occupied bricks form those values again),
+// the tables of all slots come from four launches together, and one wait for the
+// brick counts serves them all. 1024^3 with temperature, 4 mips, fp16: 31.6 -> 5.4 ms
+// against a pass per step and a wait per slot (kLevels 2.5 ms, of which reading the grid
+// once takes 0.7, the temperature's kBrickMax 0.74 = 5.8 TB/s, the fills 1.7: their
+// VALU work per value); 96^3, 3 mips: 1.72 -> 0.15 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
-#include <vector>
+#include <limits>
 
 #include "vr_launch.h"
 #include "vr_volume.h"
@@ -27,9 +38,11 @@ constexpr int kBuildThreads = 256;
 __device__ __forceinline__ size_t lin(int x, int y, int z, int nx, int ny) {
     return (size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * (size_t)z);
 }
+// A raw grid's value as the build takes it (negative and NaN to 0), 0 outside the grid.
 __device__ __forceinline__ float at(const float* __restrict__ s, int x, int y, int z, int nx, int ny, int nz) {
     if (x < 0 || y < 0 || z < 0 || x >= nx || y >= ny || z >= nz) return 0.f;
-    return s[lin(x, y, z, nx, ny)];
+    const float v = s[lin(x, y, z, nx, ny)];
+    return v > 0.f ? v : 0.f;
 }
 
 // IEEE binary16 bits of a float, round to nearest even (the host build's rule,
@@ -75,323 +88,534 @@ __device__ __forceinline__ float stored(float x, float gmax, int fp16) {
     return fp16 ? halfValue(halfBits(x)) : x;
 }
 
-// The largest of each wave's values into *maxBits (values are >= 0, so their
-// bits order as the values do).
-__device__ __forceinline__ void waveMax(unsigned m, unsigned* __restrict__ maxBits) {
-    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
-    if ((threadIdx.x & 63) == 0 && m) atomicMax(maxBits, m);
+__device__ __forceinline__ float laneMax(float m, int from, int to) {
+    for (int o = from; o <= to; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+    return m;
 }
-// out = max(in, 0); bad counts non-finite inputs; maxBits: the largest output
-__global__ __launch_bounds__(kBuildThreads) void kClamp(const float* __restrict__ in, float* __restrict__ out,
-                                                        size_t n, int* __restrict__ bad, unsigned* __restrict__ maxBits) {
-    unsigned m = 0u;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float v = in[i];
-        if (!isfinite(v)) atomicAdd(bad, 1);
-        const float o = v > 0.f ? v : 0.f;
-        out[i] = o;
-        if (isfinite(v)) m = max(m, __float_as_uint(o));
+// values are >= 0, so their bits order as the values do
+__device__ __forceinline__ void maxInto(unsigned* __restrict__ bits, float m) {
+    if (m > 0.f) atomicMax(bits, __float_as_uint(m));
+}
+// A voxel of the conservative grid: an empty voxel takes the mean of the positive
+// values of its 27-neighbourhood, summed x outermost. t: the value at an offset (>= 0).
+template <class T>
+__device__ __forceinline__ float dilated(float v, T t) {
+    if (v != 0.f) return v;
+    float avg = 0.f;
+    for (int ii = -1; ii <= 1; ii++)
+        for (int jj = -1; jj <= 1; jj++)
+            for (int kk = -1; kk <= 1; kk++) avg += t(ii, jj, kk);
+    avg /= 27.f;
+    return avg > 0.f ? avg : v;
+}
+// 2x box reduction, weight 1/8 per tap summed x-major, negative results to 0
+template <class T>
+__device__ __forceinline__ float reduced(T t) {
+    float res = 0.f;
+    for (int a = 0; a < 2; a++)
+        for (int b = 0; b < 2; b++)
+            for (int c = 0; c < 2; c++) res = __fadd_rn(res, __fmul_rn(0.125f, t(a, b, c)));
+    return res > 0.f ? res : 0.f;
+}
+
+__global__ __launch_bounds__(kBuildThreads) void kClear(unsigned* __restrict__ p, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0u;
+}
+
+// Both mip chains down to level 3 from one read of the raw grid. A workgroup takes a
+// 64 x 8 x 8 tile (8 whole bricks of mip 0, one voxel row of level 3) and its
+// one-voxel halo through LDS: the density and its dilation are formed there, reduced
+// level by level, and each level's values and bricks' largest values written. A tile
+// without a positive value (most of a sparse volume) writes its zeros and ends.
+// Tiles wider in x than the 128-byte lines they touch, 8 deep so that level 3 and the
+// bricks need no exchange between workgroups; 47 KB of LDS, three workgroups per CU.
+constexpr int kTX = 64, kTY = 8, kTZ = 8;
+constexpr int kRow = 72;  // LDS row: voxel x at 4 + x, so that 16-byte stores align
+struct LevelGrids {
+    float* out[2][4];         // level 1..3 grids of the density [0] and its dilation [1]
+    unsigned* brickMax[2][4]; // level 0..3: the largest value (bits) per brick
+};
+template <bool ALIGNED>
+__global__ __launch_bounds__(kBuildThreads) void kLevels(const float* __restrict__ s, int nx, int ny, int nz, int levels,
+                                                         LevelGrids L, int* __restrict__ bad) {
+    __shared__ __align__(16) float t[kTZ + 2][kTY + 2][kRow];
+    __shared__ float dil[kTZ][kTY][kTX];
+    __shared__ float m1[2][4][4][32], m2[2][2][2][16];
+    __shared__ float part[2][4][8];
+    const int x0 = (int)blockIdx.x * kTX, y0 = (int)blockIdx.y * kTY, z0 = (int)blockIdx.z * kTZ;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    bool positive = false, finite = true;
+    // all of a thread's loads are issued before the first is used: 3 workgroups per CU
+    // hold too few waves to cover HBM's latency otherwise (3.4 -> 2.5 ms at 1024^3)
+    constexpr int kLoads = ((kTZ + 2) * (kTY + 2) * 16 + kBuildThreads - 1) / kBuildThreads;
+    float v[kLoads][4];
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) {
+        const int i = tid + j * kBuildThreads, q = i & 15, r = i >> 4, ly = r % (kTY + 2), lz = r / (kTY + 2);
+        const int x = x0 + 4 * q, y = y0 + ly - 1, z = z0 + lz - 1;
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[j][k] = 0.f;
+        if (lz < kTZ + 2 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) {
+            const float* src = s + lin(x, y, z, nx, ny);
+            if (ALIGNED) {
+                const float4 w = *reinterpret_cast<const float4*>(src);
+                v[j][0] = w.x; v[j][1] = w.y; v[j][2] = w.z; v[j][3] = w.w;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[j][k] = src[k];
+            }
+        }
     }
-    waveMax(m, maxBits);
-}
-// kClamp on 16-byte-aligned grids whose size is a multiple of 4, four values per load
-__global__ __launch_bounds__(kBuildThreads) void kClamp4(const float4* __restrict__ in, float4* __restrict__ out,
-                                                         size_t n4, int* __restrict__ bad, unsigned* __restrict__ maxBits) {
-    unsigned m = 0u;
-    int nonFinite = 0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
-        const float4 v = in[i];
-        const float e[4] = {v.x, v.y, v.z, v.w};
-        float o[4];
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) {
+        const int i = tid + j * kBuildThreads, q = i & 15, r = i >> 4, ly = r % (kTY + 2), lz = r / (kTY + 2);
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            o[k] = e[k] > 0.f ? e[k] : 0.f;
-            if (isfinite(e[k])) m = max(m, __float_as_uint(o[k]));
-            else nonFinite++;
+            finite = finite && isfinite(v[j][k]);
+            v[j][k] = v[j][k] > 0.f ? v[j][k] : 0.f;
+            positive = positive || v[j][k] > 0.f;
         }
-        out[i] = make_float4(o[0], o[1], o[2], o[3]);
+        if (lz < kTZ + 2)
+            *reinterpret_cast<float4*>(&t[lz][ly][4 + 4 * q]) = make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
     }
-    if (nonFinite) atomicAdd(bad, nonFinite);
-    waveMax(m, maxBits);
-}
-// Conservative grid: an empty voxel takes the mean of the positive values of its
-// 27-neighbourhood (summed x outermost, as the host build does). A workgroup takes
-// a 64 x 8 x 8 tile: the tile and its one-voxel halo are read once into LDS, a tile
-// with no positive value anywhere in it is copied through, and every other empty
-// voxel sums its neighbourhood from LDS in the host build's order.
-constexpr int kDilX = 64, kDilY = 8, kDilZ = 8;
-__global__ __launch_bounds__(kBuildThreads) void kDilate(const float* __restrict__ s, float* __restrict__ d, int nx,
-                                                         int ny, int nz, unsigned* __restrict__ maxBits) {
-    constexpr int TX = kDilX + 2, TY = kDilY + 2, TZ = kDilZ + 2;
-    __shared__ float t[TZ][TY][TX];
-    const int x0 = (int)blockIdx.x * kDilX, y0 = (int)blockIdx.y * kDilY, z0 = (int)blockIdx.z * kDilZ;
-    int positive = 0;
-    for (int i = threadIdx.x; i < TX * TY * TZ; i += blockDim.x) {
-        const int lx = i % TX, ly = (i / TX) % TY, lz = i / (TX * TY);
-        const float v = at(s, x0 + lx - 1, y0 + ly - 1, z0 + lz - 1, nx, ny, nz);
-        t[lz][ly][lx] = v;
-        positive |= v > 0.f ? 1 : 0;
+    if (tid < 2 * (kTZ + 2) * (kTY + 2)) {
+        const int e = tid & 1, r = tid >> 1, ly = r % (kTY + 2), lz = r / (kTY + 2);
+        const float v = at(s, e ? x0 + kTX : x0 - 1, y0 + ly - 1, z0 + lz - 1, nx, ny, nz);
+        positive = positive || v > 0.f;
+        t[lz][ly][e ? 4 + kTX : 3] = v;
     }
-    const int any = __syncthreads_or(positive);
-    unsigned m = 0u;
-    for (int i = threadIdx.x; i < kDilX * kDilY * kDilZ; i += blockDim.x) {
-        const int lx = i % kDilX, ly = (i / kDilX) % kDilY, lz = i / (kDilX * kDilY);
-        const int x = x0 + lx, y = y0 + ly, z = z0 + lz;
-        if (x >= nx || y >= ny || z >= nz) continue;
-        const float v = t[lz + 1][ly + 1][lx + 1];
-        float o = v;
-        if (v == 0.f && any) {
-            float avg = 0.f;
-            for (int ii = -1; ii <= 1; ii++)
-                for (int jj = -1; jj <= 1; jj++)
-                    for (int kk = -1; kk <= 1; kk++) {
-                        const float tv = t[lz + 1 + kk][ly + 1 + jj][lx + 1 + ii];
-                        avg += tv > 0.f ? tv : 0.f;
-                    }
-            avg /= 27.f;
-            if (avg > 0.f) o = avg;
+    if (!finite) *bad = 1;
+    const int any = __syncthreads_or(positive ? 1 : 0);
+    const int nbx = nx / 8, nby = ny / 8, bricks = min(8, nbx - 8 * (int)blockIdx.x);
+    const size_t b0 = 8 * (size_t)blockIdx.x + (size_t)nbx * (blockIdx.y + (size_t)nby * blockIdx.z);
+    if (!any) {
+        if (tid < 2 * bricks) L.brickMax[tid / bricks][0][b0 + tid % bricks] = 0u;
+        for (int l = 1; l <= levels; l++) {
+            const int w = kTX >> l, h = kTY >> l, n = w * h * (kTZ >> l), gx = nx >> l, gy = ny >> l;
+            for (int i = tid; i < 2 * n; i += kBuildThreads) {
+                const int c = i / n, j = i % n, x = (x0 >> l) + j % w, y = (y0 >> l) + j / w % h, z = (z0 >> l) + j / w / h;
+                if (x < gx) L.out[c][l][lin(x, y, z, gx, gy)] = 0.f;
+            }
         }
-        d[lin(x, y, z, nx, ny)] = o;
-        m = max(m, __float_as_uint(o));
+        return;
     }
-    waveMax(m, maxBits);
+    // level 0: the dilation, and the largest value of each of the tile's bricks (8 lanes wide each)
+    float md = 0.f, mc = 0.f;
+    for (int r = wv; r < kTY * kTZ; r += 4) {
+        const int y = r % kTY, z = r / kTY;
+        const float v = t[z + 1][y + 1][4 + lane];
+        const float c = dilated(v, [&](int i, int j, int k) { return t[z + 1 + k][y + 1 + j][4 + lane + i]; });
+        dil[z][y][lane] = c;
+        md = fmaxf(md, v);
+        mc = fmaxf(mc, c);
+    }
+    md = laneMax(md, 1, 4);
+    mc = laneMax(mc, 1, 4);
+    if ((lane & 7) == 0) { part[0][wv][lane >> 3] = md; part[1][wv][lane >> 3] = mc; }
+    __syncthreads();
+    if (tid < 16) {
+        const int c = tid >> 3, b = tid & 7;
+        const float m = fmaxf(fmaxf(part[c][0][b], part[c][1][b]), fmaxf(part[c][2][b], part[c][3][b]));
+        if (b < bricks) L.brickMax[c][0][b0 + b] = __float_as_uint(m);
+    }
+    if (levels < 1) return;
+    // level l's bricks cover 2^l tiles a side in y and z: their maxima meet in memory
+    auto brickAtLevel = [&](int l, int bx) {
+        const int bw = (nx >> l) / 8, bh = (ny >> l) / 8;
+        return (size_t)bx + (size_t)bw * (size_t)(((y0 >> l) / 8) + (size_t)bh * ((z0 >> l) / 8));
+    };
+    {
+        const int gx = nx >> 1, gy = ny >> 1;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            float m = 0.f;
+            for (int r = wv * 2 + (lane >> 5); r < 16; r += 8) {
+                const int x = lane & 31, y = r & 3, z = r >> 2;
+                const float o = c == 0 ? reduced([&](int a, int b, int k) { return t[2 * z + k + 1][2 * y + b + 1][4 + 2 * x + a]; })
+                                       : reduced([&](int a, int b, int k) { return dil[2 * z + k][2 * y + b][2 * x + a]; });
+                m1[c][z][y][x] = o;
+                // voxels past the grid's edge are 0 and not stored
+                if (x0 / 2 + x < gx) L.out[c][1][lin(x0 / 2 + x, y0 / 2 + y, z0 / 2 + z, gx, gy)] = o;
+                if (x0 / 2 + x < gx) m = fmaxf(m, o);
+            }
+            m = laneMax(laneMax(m, 1, 4), 32, 32);
+            if (lane < 32 && (lane & 7) == 0 && m > 0.f)
+                maxInto(&L.brickMax[c][1][brickAtLevel(1, (x0 / 2 + lane) / 8)], m);
+        }
+    }
+    if (levels < 2) return;
+    __syncthreads();
+    if (tid < 128) {
+        const int c = wv, x = lane & 15, y = (lane >> 4) & 1, z = lane >> 5, gx = nx >> 2, gy = ny >> 2;
+        float o = reduced([&](int a, int b, int k) { return m1[c][2 * z + k][2 * y + b][2 * x + a]; });
+        m2[c][z][y][x] = o;
+        const bool in = x0 / 4 + x < gx;
+        if (in) L.out[c][2][lin(x0 / 4 + x, y0 / 4 + y, z0 / 4 + z, gx, gy)] = o;
+        const float m = laneMax(laneMax(in ? o : 0.f, 1, 4), 16, 32);
+        if (lane < 16 && (lane & 7) == 0) maxInto(&L.brickMax[c][2][brickAtLevel(2, min(x0 / 4 + x, gx - 1) / 8)], m);
+    }
+    if (levels < 3) return;
+    __syncthreads();
+    if (tid < 16) {
+        const int c = tid >> 3, x = tid & 7, gx = nx >> 3, gy = ny >> 3;
+        const float o = reduced([&](int a, int b, int k) { return m2[c][k][b][2 * x + a]; });
+        if (x0 / 8 + x < gx) {
+            L.out[c][3][lin(x0 / 8 + x, y0 / 8, z0 / 8, gx, gy)] = o;
+            maxInto(&L.brickMax[c][3][brickAtLevel(3, (x0 / 8 + x) / 8)], o);
+        }
+    }
 }
-// 2x box reduction, weight 1/8 per tap summed x-major, negative results to 0; d is nx/2 x ny/2 x nz/2
+
+// The largest value of every brick of a grid (negative and NaN taken as 0); one
+// workgroup per 64 x 8 x 8 tile. bad: set when a value is not finite.
+template <bool ALIGNED>
+__global__ __launch_bounds__(kBuildThreads) void kBrickMax(const float* __restrict__ s, int nx, int ny, int nz,
+                                                           unsigned* __restrict__ brickMax, int* __restrict__ bad) {
+    __shared__ float part[4][8];
+    const int x0 = (int)blockIdx.x * kTX, y0 = (int)blockIdx.y * 8, z0 = (int)blockIdx.z * 8;
+    const int q = threadIdx.x & 15, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    float m = 0.f;
+    bool finite = true;
+    if (x0 + 4 * q < nx) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = (threadIdx.x >> 4) + 16 * i;
+            const float* src = s + lin(x0 + 4 * q, y0 + (r & 7), z0 + (r >> 3), nx, ny);
+            if (ALIGNED) {
+                const float4 w = *reinterpret_cast<const float4*>(src);
+                v[4 * i] = w.x; v[4 * i + 1] = w.y; v[4 * i + 2] = w.z; v[4 * i + 3] = w.w;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[4 * i + k] = src[k];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            finite = finite && isfinite(v[i]);
+            m = fmaxf(m, v[i] > 0.f ? v[i] : 0.f);
+        }
+    }
+    if (!finite) *bad = 1;
+    m = laneMax(laneMax(m, 1, 1), 16, 32);
+    if (lane < 16 && (lane & 1) == 0) part[wv][lane >> 1] = m;
+    __syncthreads();
+    if (threadIdx.x < 8 && x0 + 8 * (int)threadIdx.x < nx) {
+        const int b = threadIdx.x;
+        m = fmaxf(fmaxf(part[0][b], part[1][b]), fmaxf(part[2][b], part[3][b]));
+        brickMax[x0 / 8 + b + (size_t)(nx / 8) * (blockIdx.y + (size_t)(ny / 8) * blockIdx.z)] = __float_as_uint(m);
+    }
+}
+// One 2x reduction of a whole grid (levels past kLevels'); d is nx/2 x ny/2 x nz/2
 __global__ __launch_bounds__(kBuildThreads) void kReduce2(const float* __restrict__ s, float* __restrict__ d, int nx,
-                                                          int ny, int nz, unsigned* __restrict__ maxBits) {
+                                                          int ny, int nz) {
     const int dx = nx / 2, dy = ny / 2, dz = nz / 2;
     const size_t n = (size_t)dx * dy * dz;
-    unsigned m = 0u;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         const int x = (int)(i % dx), y = (int)((i / dx) % dy), z = (int)(i / ((size_t)dx * dy));
-        float res = 0.f;
-        for (int a = 0; a < 2; a++)
-            for (int b = 0; b < 2; b++)
-                for (int c = 0; c < 2; c++)
-                    res = __fadd_rn(res, __fmul_rn(0.125f, s[lin(2 * x + a, 2 * y + b, 2 * z + c, nx, ny)]));
-        const float o = res > 0.f ? res : 0.f;
-        d[i] = o;
-        m = max(m, __float_as_uint(o));
-    }
-    waveMax(m, maxBits);
-}
-// per brick cell: does any stored value of its 8^3 voxels exceed 0
-__global__ __launch_bounds__(kBuildThreads) void kBrickOcc(const float* __restrict__ s, int nx, int ny, int nz,
-                                                           int nbx, int nby, int nbz, const unsigned* __restrict__ gmaxBits,
-                                                           int fp16, uint8_t* __restrict__ occ) {
-    const float gmax = __uint_as_float(*gmaxBits);
-    const size_t nb = (size_t)nbx * nby * nbz;
-    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < nb; c += (size_t)gridDim.x * blockDim.x) {
-        const int bx = (int)(c % nbx), by = (int)((c / nbx) % nby), bz = (int)(c / ((size_t)nbx * nby));
-        bool any = false;
-        // a row's 8 loads are issued together, then tested
-        for (int z = 0; z < 8 && !any; z++)
-            for (int y = 0; y < 8 && !any; y++) {
-                float row[8];
-                const float* src = s + lin(bx * 8, by * 8 + y, bz * 8 + z, nx, ny);
-#pragma unroll
-                for (int x = 0; x < 8; x++) row[x] = src[x];
-#pragma unroll
-                for (int x = 0; x < 8; x++) any |= stored(row[x], gmax, fp16) > 0.f;
-            }
-        occ[c] = any ? 1 : 0;
+        d[i] = reduced([&](int a, int b, int c) { return s[lin(2 * x + a, 2 * y + b, 2 * z + c, nx, ny)]; });
     }
 }
-// occupancy words {bits, prefix}: the bits here, the counts for the scan
-__global__ __launch_bounds__(kBuildThreads) void kOccWords(const uint8_t* __restrict__ occ, size_t nb,
-                                                           uint32_t* __restrict__ words, uint32_t* __restrict__ cnt,
-                                                           size_t nw) {
-    for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += (size_t)gridDim.x * blockDim.x) {
-        uint32_t bits = 0u;
-        for (int b = 0; b < 32; b++) {
-            const size_t c = w * 32 + b;
-            if (c < nb && occ[c]) bits |= 1u << b;
+
+// The tables of every slot of a frame, blockIdx.y = slot: the grid's largest value,
+// the occupancy words, their prefix sums, the brick ids and the block table.
+struct TableJobs {
+    BuildGrid g[kFrameSlots];
+    BuildStats* stats;
+};
+__global__ __launch_bounds__(kBuildThreads) void kGridMax(const TableJobs J) {
+    const BuildGrid& g = J.g[blockIdx.y];
+    float m = 0.f;
+    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < g.cells; c += (size_t)gridDim.x * blockDim.x)
+        m = fmaxf(m, __uint_as_float(g.brickMax[c]));
+    m = laneMax(m, 1, 32);
+    if ((threadIdx.x & 63) == 0) maxInto(&J.stats->maxBits[blockIdx.y], m);
+}
+// Occupancy: does a brick hold a value that its stored form keeps above 0? Storing is
+// monotone, so its largest value tells. Also clears the block table.
+__global__ __launch_bounds__(kBuildThreads) void kWords(const TableJobs J, int fp16) {
+    const BuildGrid& g = J.g[blockIdx.y];
+    const float gmax = __uint_as_float(J.stats->maxBits[blockIdx.y]);
+    const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = i0; i < g.blocks; i += stride) g.nodes[i] = 0u;
+    // whole waves iterate together: 64 cells are two words
+    for (size_t c = i0; c - (threadIdx.x & 63) < g.cells; c += stride) {
+        const bool occ = c < g.cells && stored(__uint_as_float(g.brickMax[c]), gmax, fp16) > 0.f;
+        const uint64_t bits = __ballot(occ);
+        const int l = threadIdx.x & 63;
+        if ((l & 31) == 0 && c < g.cells) g.words[2 * (c / 32)] = (uint32_t)(l ? bits >> 32 : bits);
+    }
+}
+// Exclusive prefix of the words' popcounts into their second entries, one workgroup a
+// slot: 4096 consecutive words an iteration, scanned by wave and then across the waves.
+__global__ __launch_bounds__(1024) void kScanWords(const TableJobs J) {
+    const BuildGrid& g = J.g[blockIdx.y];
+    __shared__ uint32_t waveSum[16];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const size_t nw = (g.cells + 31) / 32;
+    uint32_t base = 0u;
+    for (size_t w0 = 0; w0 < nw; w0 += 4096) {
+        const size_t w = w0 + 4 * threadIdx.x;
+        uint32_t n[4], sum = 0u;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            n[k] = w + k < nw ? (uint32_t)__popc(g.words[2 * (w + k)]) : 0u;
+            sum += n[k];
         }
-        words[2 * w] = bits;
-        cnt[w] = (uint32_t)__popc(bits);
-    }
-}
-// Exclusive prefix of cnt into the words' second entries, one workgroup: each
-// thread sums a contiguous run, the runs' totals are scanned in LDS, then each
-// thread writes its run. total receives the number of bricks.
-__global__ __launch_bounds__(1024) void kScanWords(uint32_t* __restrict__ words, const uint32_t* __restrict__ cnt,
-                                                   size_t nw, uint32_t* __restrict__ total) {
-    __shared__ uint32_t part[1024];
-    const size_t per = (nw + 1023) / 1024;
-    const size_t w0 = threadIdx.x * per, w1 = min(nw, w0 + per);
-    uint32_t s = 0u;
-    for (size_t w = w0; w < w1; w++) s += cnt[w];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const uint32_t v = threadIdx.x >= (unsigned)o ? part[threadIdx.x - o] : 0u;
+        uint32_t incl = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, o);
+            if (lane >= o) incl += y;
+        }
+        if (lane == 63) waveSum[wv] = incl;
         __syncthreads();
-        part[threadIdx.x] += v;
+        uint32_t before = base, all = base;
+        for (int k = 0; k < 16; k++) {
+            if (k < wv) before += waveSum[k];
+            all += waveSum[k];
+        }
+        before += incl - sum;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (w + k < nw) g.words[2 * (w + k) + 1] = before;
+            before += n[k];
+        }
+        base = all;
         __syncthreads();
     }
-    uint32_t run = part[threadIdx.x] - s;
-    for (size_t w = w0; w < w1; w++) {
-        words[2 * w + 1] = run;
-        run += cnt[w];
-    }
-    if (threadIdx.x == 1023) *total = part[1023];
+    if (threadIdx.x == 0) J.stats->count[blockIdx.y] = base;
 }
-// brick ids in brick-table order: the table, each id's cell, the block table
-__global__ __launch_bounds__(kBuildThreads) void kBrickIds(const uint32_t* __restrict__ words, int nbx, int nby,
-                                                           int nbz, int nnx, int nny, uint32_t* __restrict__ table,
-                                                           uint32_t* __restrict__ cellOf,
-                                                           uint32_t* __restrict__ nodes) {
-    const size_t nb = (size_t)nbx * nby * nbz;
-    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < nb; c += (size_t)gridDim.x * blockDim.x) {
-        const uint32_t bits = words[2 * (c / 32)], b = (uint32_t)(c % 32);
-        if (!((bits >> b) & 1u)) { table[c] = kEmpty; continue; }
-        const uint32_t id = words[2 * (c / 32) + 1] + (uint32_t)__popc(bits & ((1u << b) - 1u));
-        table[c] = id;
-        cellOf[id] = (uint32_t)c;
-        const int bx = (int)(c % nbx), by = (int)((c / nbx) % nby), bz = (int)(c / ((size_t)nbx * nby));
-        atomicOr(&nodes[(bx / 16) + (size_t)nnx * ((by / 16) + (size_t)nny * (bz / 16))], 1u);
+__global__ __launch_bounds__(kBuildThreads) void kBrickIds(const TableJobs J) {
+    const BuildGrid& g = J.g[blockIdx.y];
+    const uint32_t nbx = g.nx / 8, nby = g.ny / 8;
+    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < g.cells; c += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t bits = g.words[2 * (c / 32)], b = (uint32_t)(c % 32);
+        if (!((bits >> b) & 1u)) { g.table[c] = kEmpty; continue; }
+        const uint32_t id = g.words[2 * (c / 32) + 1] + (uint32_t)__popc(bits & ((1u << b) - 1u));
+        g.table[c] = id;
+        g.cellOf[id] = (uint32_t)c;
+        const uint32_t r = (uint32_t)c / nbx, bx = (uint32_t)c % nbx, by = r % nby, bz = r / nby;
+        g.nodes[(bx / 16) + (size_t)g.nnx * ((by / 16) + (size_t)g.nny * (bz / 16))] = 1u;
     }
 }
-// per brick: its 10^3 apron values (stored form) and bounds {min, max, sum / 512, 0}
-template <int FP16>
-__global__ __launch_bounds__(kBuildThreads) void kBrickFill(const float* __restrict__ s, int nx, int ny, int nz,
-                                                            int nbx, int nby, const uint32_t* __restrict__ cellOf,
-                                                            const uint32_t* __restrict__ count,
-                                                            const unsigned* __restrict__ gmaxBits,
-                                                            void* __restrict__ pool, float* __restrict__ bounds) {
-    const float gmax = __uint_as_float(*gmaxBits);
-    const uint32_t nbricks = *count;
-    for (size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x; id < nbricks;
-         id += (size_t)gridDim.x * blockDim.x) {
-        const uint32_t c = cellOf[id];
-        const int x0 = (int)(c % nbx) * 8, y0 = (int)((c / nbx) % nby) * 8, z0 = (int)(c / ((size_t)nbx * nby)) * 8;
-        float mn = 3.402823466e+38f, mx = 0.f, sum = 0.f;
-        for (int i = -1; i <= 8; i++)
-            for (int j = -1; j <= 8; j++) {
-                // the 10 loads along z are issued together, then consumed in order
-                float raw[kApron];
+
+// Per brick its 10^3 apron values (stored form) and bounds {min, max, sum / 512, 0}.
+// A wave fills a brick: 16 values a lane, rows of the source read along x. The
+// bounds' sum runs over the apron with x outermost, one add after the other, as the
+// host's: the values go through LDS in that order and one lane a brick adds them,
+// 4 bricks side by side. DIL: the bricks of the dilated raw grid, whose values are
+// formed from a 12^3 region in LDS.
+struct FillJobs {
+    int n;
+    int start[kFrameSlots + 1];  // first workgroup of each slot
+    uint32_t count[kFrameSlots];
+    float least[kFrameSlots];    // the smallest value whose stored form is not clamped to 0
+    BuildGrid g[kFrameSlots];
+};
+// The smallest x with x / gmax >= 1e-9 (stored()'s clamp; the quotient is monotone in x):
+// a compare per value in place of a division.
+float leastKept(float gmax) {
+    if (!(gmax > 0.f)) return std::numeric_limits<float>::infinity();
+    float x = 1e-9f * gmax;
+    while (x > 0.f && x / gmax >= 1e-9f) x = std::nextafter(x, 0.f);
+    while (x / gmax < 1e-9f) x = std::nextafter(x, gmax);
+    return x;
+}
+constexpr int kFillBricks = 4, kFillRow = 1004;
+template <int FP16, bool DIL>
+__global__ __launch_bounds__(64 * kFillBricks) void kBrickFill(const FillJobs J) {
+    __shared__ __align__(16) float vals[kFillBricks][kFillRow];
+    __shared__ float raw[DIL ? kFillBricks : 1][DIL ? 1728 : 1];
+    int i = 0;
+    while (i + 1 < J.n && (int)blockIdx.x >= J.start[i + 1]) i++;
+    const BuildGrid& g = J.g[i];
+    const float least = J.least[i];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const size_t id0 = (size_t)((int)blockIdx.x - J.start[i]) * kFillBricks, id = id0 + wv;
+    const bool live = id < J.count[i];
+    const uint32_t nbx = g.nx / 8, nby = g.ny / 8, c = live ? g.cellOf[id] : 0u;
+    const int x0 = (int)(c % nbx) * 8, y0 = (int)(c / nbx % nby) * 8, z0 = (int)(c / nbx / nby) * 8;
+    if constexpr (DIL) {
+        if (live) {
+            float r[27];
 #pragma unroll
-                for (int k = -1; k <= 8; k++) raw[k + 1] = at(s, x0 + i, y0 + j, z0 + k, nx, ny, nz);
+            for (int k = 0; k < 27; k++) {
+                const int v = lane + 64 * k;
+                r[k] = at(g.src, x0 + v % 12 - 2, y0 + v / 12 % 12 - 2, z0 + v / 144 - 2, g.nx, g.ny, g.nz);
+            }
 #pragma unroll
-                for (int k = -1; k <= 8; k++) {
-                    const float v = stored(raw[k + 1], gmax, FP16);
-                    const size_t o = id * kBrickVals + (size_t)(i + 1) + kApron * ((size_t)(j + 1) + kApron * (size_t)(k + 1));
-                    if (FP16) ((uint16_t*)pool)[o] = halfBits(v);
-                    else ((float*)pool)[o] = v;
-                    mn = fminf(mn, v);
-                    mx = fmaxf(mx, v);
-                    sum = __fadd_rn(sum, v);
+            for (int k = 0; k < 27; k++) raw[wv][lane + 64 * k] = r[k];
+        }
+        __syncthreads();
+    }
+    float mn = 3.402823466e+38f, mx = 0.f;
+    if (live) {
+        // two neighbours along x a lane: one 4-byte store of an fp16 pair. The loads of all
+        // of a lane's values are issued together
+        constexpr int kPairs = (kBrickVals / 2 + 63) / 64;
+        float r[kPairs][2];
+#pragma unroll
+        for (int j = 0; j < kPairs; j++) {
+            const int v = 2 * lane + 128 * j, a = v % kApron, b = v / kApron % kApron, d = v / (kApron * kApron);
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int x = x0 + a + e - 1, y = y0 + b - 1, z = z0 + d - 1;
+                if (v >= kBrickVals) r[j][e] = 0.f;
+                else if constexpr (DIL) {
+                    const bool in = x >= 0 && y >= 0 && z >= 0 && x < g.nx && y < g.ny && z < g.nz;
+                    const float* t = &raw[wv][(a + e + 1) + 12 * ((b + 1) + 12 * (d + 1))];
+                    r[j][e] = in ? dilated(t[0], [&](int ii, int jj, int kk) { return t[ii + 12 * (jj + 12 * kk)]; }) : 0.f;
+                } else {
+                    r[j][e] = at(g.src, x, y, z, g.nx, g.ny, g.nz);
                 }
             }
-        bounds[4 * id + 0] = mn;
-        bounds[4 * id + 1] = mx;
-        bounds[4 * id + 2] = sum / 512.f;
-        bounds[4 * id + 3] = 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < kPairs; j++) {
+            const int v = 2 * lane + 128 * j, a = v % kApron, b = v / kApron % kApron, d = v / (kApron * kApron);
+            if (v >= kBrickVals) continue;
+            // stored() by the conversion unit: round to nearest even, overflow to infinity and
+            // subnormals kept, as halfBits rounds (values here are finite and >= 0)
+            float o[2];
+            uint16_t hb[2];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                o[e] = r[j][e] < least ? 0.f : r[j][e];
+                if (FP16) {
+                    const _Float16 h = (_Float16)o[e];
+                    hb[e] = __builtin_bit_cast(uint16_t, h);
+                    o[e] = (float)h;
+                }
+                vals[wv][(a + e) * 100 + b * 10 + d] = o[e];
+                mn = fminf(mn, o[e]);
+                mx = fmaxf(mx, o[e]);
+            }
+            if (FP16)
+                reinterpret_cast<uint32_t*>((uint16_t*)g.pool + id * kBrickVals)[v / 2] =
+                    (uint32_t)hb[0] | (uint32_t)hb[1] << 16;
+            else
+                reinterpret_cast<float2*>((float*)g.pool + id * kBrickVals)[v / 2] = make_float2(o[0], o[1]);
+        }
+        for (int o = 1; o < 64; o <<= 1) {
+            mn = fminf(mn, __shfl_xor(mn, o));
+            mx = fmaxf(mx, __shfl_xor(mx, o));
+        }
+        if (lane == 0) {
+            g.bounds[4 * id + 0] = mn;
+            g.bounds[4 * id + 1] = mx;
+            g.bounds[4 * id + 3] = 0.f;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kFillBricks && id0 + threadIdx.x < J.count[i]) {
+        const float4* v = reinterpret_cast<const float4*>(vals[threadIdx.x]);
+        float sum = 0.f;
+#pragma unroll 10
+        for (int k = 0; k < kBrickVals / 4; k++) {
+            const float4 q = v[k];
+            sum = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(sum, q.x), q.y), q.z), q.w);
+        }
+        g.bounds[4 * (id0 + threadIdx.x) + 2] = sum / 512.f;
     }
 }
 
 dim3 gridFor(size_t n) { return dim3((unsigned)std::min<size_t>((n + kBuildThreads - 1) / kBuildThreads, 65536)); }
+bool aligned16(const void* p) { return ((uintptr_t)p % 16) == 0; }
+dim3 tileGrid(int nx, int ny, int nz) { return dim3((unsigned)((nx + kTX - 1) / kTX), (unsigned)(ny / 8), (unsigned)(nz / 8)); }
 
 }  // namespace
 
-hipError_t buildClamp(hipStream_t st, const float* in, float* out, size_t n, int* bad, unsigned* maxBits) {
-    if (n % 4 == 0 && ((uintptr_t)in % 16) == 0 && ((uintptr_t)out % 16) == 0)
-        hipLaunchKernelGGL(kClamp4, gridFor(n / 4), dim3(kBuildThreads), 0, st, (const float4*)in, (float4*)out, n / 4,
-                           bad, maxBits);
+hipError_t buildClear(hipStream_t st, void* p, size_t words) {
+    hipLaunchKernelGGL(kClear, gridFor(words), dim3(kBuildThreads), 0, st, (unsigned*)p, words);
+    return hipGetLastError();
+}
+hipError_t buildLevels(hipStream_t st, const float* s, int nx, int ny, int nz, int levels, float* const out[2][4],
+                       unsigned* const brickMax[2][4], int* bad) {
+    LevelGrids L;
+    for (int c = 0; c < 2; c++)
+        for (int l = 0; l < 4; l++) { L.out[c][l] = out[c][l]; L.brickMax[c][l] = brickMax[c][l]; }
+    if (aligned16(s))
+        hipLaunchKernelGGL(kLevels<true>, tileGrid(nx, ny, nz), dim3(kBuildThreads), 0, st, s, nx, ny, nz, levels, L, bad);
     else
-        hipLaunchKernelGGL(kClamp, gridFor(n), dim3(kBuildThreads), 0, st, in, out, n, bad, maxBits);
+        hipLaunchKernelGGL(kLevels<false>, tileGrid(nx, ny, nz), dim3(kBuildThreads), 0, st, s, nx, ny, nz, levels, L, bad);
     return hipGetLastError();
 }
-hipError_t buildDilate(hipStream_t st, const float* s, float* d, int nx, int ny, int nz, unsigned* maxBits) {
-    const dim3 g((unsigned)((nx + kDilX - 1) / kDilX), (unsigned)((ny + kDilY - 1) / kDilY),
-                 (unsigned)((nz + kDilZ - 1) / kDilZ));
-    hipLaunchKernelGGL(kDilate, g, dim3(kBuildThreads), 0, st, s, d, nx, ny, nz, maxBits);
+hipError_t buildBrickMax(hipStream_t st, const float* s, int nx, int ny, int nz, unsigned* brickMax, int* bad) {
+    if (aligned16(s))
+        hipLaunchKernelGGL(kBrickMax<true>, tileGrid(nx, ny, nz), dim3(kBuildThreads), 0, st, s, nx, ny, nz, brickMax, bad);
+    else
+        hipLaunchKernelGGL(kBrickMax<false>, tileGrid(nx, ny, nz), dim3(kBuildThreads), 0, st, s, nx, ny, nz, brickMax, bad);
     return hipGetLastError();
 }
-hipError_t buildReduce2(hipStream_t st, const float* s, float* d, int nx, int ny, int nz, unsigned* maxBits) {
-    hipLaunchKernelGGL(kReduce2, gridFor((size_t)(nx / 2) * (ny / 2) * (nz / 2)), dim3(kBuildThreads), 0, st, s, d,
-                       nx, ny, nz, maxBits);
+hipError_t buildReduce2(hipStream_t st, const float* s, float* d, int nx, int ny, int nz) {
+    hipLaunchKernelGGL(kReduce2, gridFor((size_t)(nx / 2) * (ny / 2) * (nz / 2)), dim3(kBuildThreads), 0, st, s, d, nx,
+                       ny, nz);
     return hipGetLastError();
 }
-
-// One slot from a dense device grid (nx, ny, nz multiples of 8, values >= 0)
-// whose largest value's bits are at gmaxBits (device memory, left there by the
-// kernel that made the grid). scratch: a device buffer of at least
-// buildScratchBytes(nx, ny, nz) bytes.
-// The slot's buffers come from allocBuf (which may hand back a buffer of an
-// earlier build); the host-side metadata goes to numBricks / maxValue.
-// Synchronises the stream (the brick count sizes the pool).
-size_t buildScratchBytes(int nx, int ny, int nz) {
-    const size_t nb = (size_t)(nx / 8) * (ny / 8) * (nz / 8), nw = (nb + 31) / 32;
-    return 256 + nb + 4 * nw + 4 * nb + 256;
-}
-hipError_t buildSlotDevice(hipStream_t st, const float* dense, int nx, int ny, int nz, const unsigned* gmaxBits,
-                           bool fp16, void* scratch, Grid& G, uint32_t& numBricks, float& maxValue,
-                           const BuildAlloc& allocBuf) {
-    hipError_t e;
-    const int nbx = nx / 8, nby = ny / 8, nbz = nz / 8;
-    const int nnx = (nbx + 15) / 16, nny = (nby + 15) / 16, nnz = (nbz + 15) / 16;
-    const size_t n = (size_t)nx * ny * nz, nb = (size_t)nbx * nby * nbz, nw = (nb + 31) / 32;
-    char* sp = (char*)scratch;
-    uint32_t* count = (uint32_t*)sp;                     // the brick count
-    uint8_t* occ = (uint8_t*)(sp + 256);
-    uint32_t* cnt = (uint32_t*)(sp + 256 + ((nb + 255) / 256) * 256);
-    uint32_t* cellOf = cnt + nw;
-    uint32_t *table, *nodes, *words;
-    if ((e = allocBuf(kBufTable, nb * 4, (void**)&table)) != hipSuccess) return e;
-    if ((e = allocBuf(kBufNodes, (size_t)nnx * nny * nnz * 4, (void**)&nodes)) != hipSuccess) return e;
-    if ((e = allocBuf(kBufWords, nw * 8, (void**)&words)) != hipSuccess) return e;
-    if ((e = hipMemsetAsync(nodes, 0, (size_t)nnx * nny * nnz * 4, st)) != hipSuccess) return e;
-    hipLaunchKernelGGL(kBrickOcc, gridFor(nb), dim3(kBuildThreads), 0, st, dense, nx, ny, nz, nbx, nby, nbz, gmaxBits,
-                       fp16 ? 1 : 0, occ);
-    hipLaunchKernelGGL(kOccWords, gridFor(nw), dim3(kBuildThreads), 0, st, occ, nb, words, cnt, nw);
-    hipLaunchKernelGGL(kScanWords, dim3(1), dim3(1024), 0, st, words, cnt, nw, count);
-    hipLaunchKernelGGL(kBrickIds, gridFor(nb), dim3(kBuildThreads), 0, st, words, nbx, nby, nbz, nnx, nny, table,
-                       cellOf, nodes);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    // one wait per slot: the brick count sizes the pool (the maximum comes along)
-    uint32_t nbr = 0;
-    unsigned hostMax = 0;
-    if ((e = hipMemcpyAsync(&nbr, count, 4, hipMemcpyDeviceToHost, st)) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(&hostMax, gmaxBits, 4, hipMemcpyDeviceToHost, st)) != hipSuccess) return e;
-    if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-    float gmax;
-    std::memcpy(&gmax, &hostMax, 4);
-    float* bounds;
-    void* pool;
-    if ((e = allocBuf(kBufBounds, (size_t)nbr * 16, (void**)&bounds)) != hipSuccess) return e;
-    if ((e = allocBuf(kBufPool, (size_t)nbr * kBrickVals * (fp16 ? 2 : 4), &pool)) != hipSuccess) return e;
-    if (nbr > 0) {
-        if (fp16)
-            hipLaunchKernelGGL(kBrickFill<1>, gridFor(nbr), dim3(kBuildThreads), 0, st, dense, nx, ny, nz, nbx, nby,
-                               cellOf, count, gmaxBits, pool, bounds);
-        else
-            hipLaunchKernelGGL(kBrickFill<0>, gridFor(nbr), dim3(kBuildThreads), 0, st, dense, nx, ny, nz, nbx, nby,
-                               cellOf, count, gmaxBits, pool, bounds);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+hipError_t buildTables(hipStream_t st, const BuildGrid* grids, int n, bool fp16, BuildStats* stats) {
+    if (n < 1 || n > kFrameSlots) return hipErrorInvalidValue;
+    TableJobs J{};
+    J.stats = stats;
+    size_t cells = 0;
+    for (int i = 0; i < n; i++) {
+        J.g[i] = grids[i];
+        cells = std::max(cells, grids[i].cells);
     }
+    const dim3 g((unsigned)std::min<size_t>((cells + kBuildThreads - 1) / kBuildThreads, 512), n);
+    hipLaunchKernelGGL(kGridMax, g, dim3(kBuildThreads), 0, st, J);
+    hipLaunchKernelGGL(kWords, g, dim3(kBuildThreads), 0, st, J, fp16 ? 1 : 0);
+    hipLaunchKernelGGL(kScanWords, dim3(1, n), dim3(1024), 0, st, J);
+    hipLaunchKernelGGL(kBrickIds, g, dim3(kBuildThreads), 0, st, J);
+    return hipGetLastError();
+}
+hipError_t buildFill(hipStream_t st, const BuildGrid* grids, const BuildStats& stats, int n, bool fp16) {
+    if (n < 1 || n > kFrameSlots) return hipErrorInvalidValue;
+    for (int dil = 0; dil < 2; dil++) {
+        FillJobs J{};
+        for (int i = 0; i < n; i++) {
+            if (grids[i].dilate != (dil != 0) || stats.count[i] == 0) continue;
+            const int k = J.n++;
+            J.g[k] = grids[i];
+            J.count[k] = stats.count[i];
+            float gmax;
+            std::memcpy(&gmax, &stats.maxBits[i], 4);
+            J.least[k] = leastKept(gmax);
+            J.start[k + 1] = J.start[k] + (int)((stats.count[i] + kFillBricks - 1) / kFillBricks);
+        }
+        if (J.n == 0) continue;
+        const dim3 g((unsigned)J.start[J.n]), blk(64 * kFillBricks);
+        if (fp16 && dil) hipLaunchKernelGGL((kBrickFill<1, true>), g, blk, 0, st, J);
+        else if (fp16) hipLaunchKernelGGL((kBrickFill<1, false>), g, blk, 0, st, J);
+        else if (dil) hipLaunchKernelGGL((kBrickFill<0, true>), g, blk, 0, st, J);
+        else hipLaunchKernelGGL((kBrickFill<0, false>), g, blk, 0, st, J);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+// The slot's descriptor once its buffers are filled (w2i is the caller's)
+void buildDescribe(const BuildGrid& b, const BuildStats& stats, int i, bool fp16, Grid& G) {
+    float gmax;
+    std::memcpy(&gmax, &stats.maxBits[i], 4);
     // the stored form of the maximum (monotone, so the largest stored value)
     float mv = gmax;
     if (!(gmax > 0.f)) mv = 0.f;
     else if (fp16) mv = halfBitsToFloat(floatToHalfBits(gmax));
     std::memset(&G, 0, sizeof(Grid));
-    G.brickTable = table;
-    G.nodeTable = nodes;
-    G.occ = words;
-    G.occWords = (int32_t)nw;
-    G.numBricks = nbr;
-    G.bounds = bounds;
-    G.pool = pool;
-    G.nbx = nbx; G.nby = nby; G.nbz = nbz;
-    G.nnx = nnx; G.nny = nny; G.nnz = nnz;
-    G.bmax[0] = (float)nx; G.bmax[1] = (float)ny; G.bmax[2] = (float)nz;
+    G.brickTable = b.table;
+    G.nodeTable = b.nodes;
+    G.occ = b.words;
+    G.occWords = (int32_t)((b.cells + 31) / 32);
+    G.numBricks = stats.count[i];
+    G.bounds = b.bounds;
+    G.pool = b.pool;
+    G.nbx = b.nx / 8; G.nby = b.ny / 8; G.nbz = b.nz / 8;
+    G.nnx = b.nnx; G.nny = b.nny; G.nnz = b.nnz;
+    G.bmax[0] = (float)b.nx; G.bmax[1] = (float)b.ny; G.bmax[2] = (float)b.nz;
     G.maxValue = mv;
     G.fp16 = fp16 ? 1 : 0;
     G.channels = 1;
     G.valid = 1;
-    numBricks = nbr;
-    maxValue = mv;
-    return hipSuccess;
 }
 
 }  // namespace vr

@@ -2,7 +2,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <functional>
 #include <vector>
 
 #include "vr_types.h"
@@ -111,22 +110,42 @@ hipError_t launchLearnedReduce(hipStream_t st, const float* partial, int waves, 
                                float* m, float* v, float lr, float c1, float c2, float* stats, int* inUse, bool judge,
                                int step);
 hipError_t launchLearnedPack(hipStream_t st, const float* prm, uint4* frags);
-// Volume grids built on the GPU from dense device grids (vr_k_build.hip): the
-// host build's clamp, conservative dilation and 2x reduction, and one slot
-// (tables, occupancy words, pool, bounds) from a dense grid. buildSlotDevice
-// appends its allocations to allocs and synchronises the stream.
-// Each also leaves the largest value it writes (as float bits, via atomicMax) at maxBits.
-hipError_t buildClamp(hipStream_t st, const float* in, float* out, size_t n, int* bad, unsigned* maxBits);
-hipError_t buildDilate(hipStream_t st, const float* s, float* d, int nx, int ny, int nz, unsigned* maxBits);
-hipError_t buildReduce2(hipStream_t st, const float* s, float* d, int nx, int ny, int nz, unsigned* maxBits);
-size_t buildScratchBytes(int nx, int ny, int nz);
-// A slot's device buffer of at least `bytes` (kind: one of kBuf*), possibly one
-// kept from an earlier build of the same slot.
+// Volume grids built on the GPU from dense device grids (vr_k_build.hip), value for
+// value as the host build makes them. One slot of the frame: its source grid (a level
+// grid, or a raw grid whose negative values count as 0; dilate: the conservative form
+// of the raw grid, formed on the fly), sizes, tables and, once the brick counts are
+// known, bounds and pool.
+struct BuildGrid {
+    const float* src;
+    int nx, ny, nz, nnx, nny, nnz;  // voxels (multiples of 8) and 128^3 blocks
+    size_t cells, blocks;           // 8^3 brick cells and 128^3 blocks
+    bool dilate;
+    unsigned* brickMax;             // scratch: the largest value per cell, as float bits
+    uint32_t* cellOf;               // scratch: the cell of each brick
+    uint32_t *table, *nodes, *words;
+    float* bounds;
+    void* pool;
+};
+// Per slot: the grid's largest value (float bits) and its bricks; non-finite inputs seen.
+struct BuildStats {
+    unsigned maxBits[kFrameSlots];
+    uint32_t count[kFrameSlots];
+    int bad[2];
+};
+hipError_t buildClear(hipStream_t st, void* p, size_t words);
+// Levels 1..levels (<= 3) of the density [0] and its dilation [1], and every brick's
+// largest value at levels 0..levels; brickMax of levels >= 1 must be zero before.
+hipError_t buildLevels(hipStream_t st, const float* s, int nx, int ny, int nz, int levels, float* const out[2][4],
+                       unsigned* const brickMax[2][4], int* bad);
+hipError_t buildBrickMax(hipStream_t st, const float* s, int nx, int ny, int nz, unsigned* brickMax, int* bad);
+hipError_t buildReduce2(hipStream_t st, const float* s, float* d, int nx, int ny, int nz);
+// Tables of n slots from their brickMax; leaves maxBits and count in stats (device, zero before).
+hipError_t buildTables(hipStream_t st, const BuildGrid* grids, int n, bool fp16, BuildStats* stats);
+// Pools and bounds of n slots; stats: buildTables' on the host.
+hipError_t buildFill(hipStream_t st, const BuildGrid* grids, const BuildStats& stats, int n, bool fp16);
+void buildDescribe(const BuildGrid& b, const BuildStats& stats, int i, bool fp16, Grid& G);
+// A slot's device buffers, kept from one build to the next.
 enum { kBufTable = 0, kBufNodes, kBufWords, kBufBounds, kBufPool, kBufKinds };
-using BuildAlloc = std::function<hipError_t(int kind, size_t bytes, void** p)>;
-hipError_t buildSlotDevice(hipStream_t st, const float* dense, int nx, int ny, int nz, const unsigned* gmaxBits,
-                           bool fp16, void* scratch, Grid& G, uint32_t& numBricks, float& maxValue,
-                           const BuildAlloc& allocBuf);
 // Importance mip chain of a lat-long map: level k of dim >> k texels at imp + off[k].
 hipError_t launchEnvImportance(hipStream_t st, const float* tex, int W, int H, float* imp, const int* off, int dim,
                                int spp);
