@@ -199,10 +199,11 @@ def test_shared_volume_renders_like_an_own_copy():
 
 @pytest.mark.parametrize("dims,mips,fp16,offset", [
     ((8, 8, 8), 1, False, 0), ((24, 40, 56), 1, True, 1), ((80, 16, 48), 2, False, 3), ((160, 32, 96), 3, True, 0),
-    ((64, 64, 192), 4, False, 2), ((128, 256, 128), 5, True, 0)])
+    ((64, 64, 192), 4, False, 2), ((128, 256, 128), 5, True, 0), ((512, 520, 64), 1, True, 0)])
 def test_device_build_at_tile_edges_equals_host_build(dims, mips, fp16, offset):
     """Grids whose sides leave remainders of the build's 64 x 8 x 8 tiles, every number of
-    levels on both sides of those the tile pass reduces, a source that is not 16-byte
+    levels on both sides of those the tile pass reduces, slots on both sides of the
+    one-workgroup table pass (32768 bricks), a source that is not 16-byte
     aligned (offset floats into an allocation), voxels at the faces, negative values and
     values below the stored clamp. The residual-ratio tracker reads the bricks' bounds."""
     import torch

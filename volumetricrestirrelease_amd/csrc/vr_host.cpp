@@ -408,6 +408,36 @@ static int uploadScene(vrestir_handle* h) {
     return VRESTIR_OK;
 }
 
+// Grid::ahead of a brick table: the groups that hold a brick, then per axis every octant
+// gathers from the side its rays move to.
+static int aheadTable(const std::vector<uint32_t>& table, int nbx, int nby, int nbz, std::vector<uint8_t>& out) {
+    const int s = aheadShiftFor(nbx, nby, nbz);
+    const int n[3] = {((nbx - 1) >> s) + 1, ((nby - 1) >> s) + 1, ((nbz - 1) >> s) + 1};
+    const int step[3] = {1, n[0], n[0] * n[1]};
+    out.assign(kAheadBytes, 0);
+    size_t c = 0;
+    for (int z = 0; z < nbz; z++)
+        for (int y = 0; y < nby; y++)
+            for (int x = 0; x < nbx; x++, c++)
+                if (table[c] != kEmpty) out[(x >> s) * step[0] + (y >> s) * step[1] + (z >> s) * step[2]] = 0xFF;
+    for (int a = 0; a < 3; a++) {
+        const int b = a == 0 ? 1 : 0, d = a == 2 ? 1 : 2;
+        for (int j = 0; j < n[b]; j++)
+            for (int k = 0; k < n[d]; k++)
+                for (int up = 0; up < 2; up++) {
+                    uint8_t mask = 0, m = 0;
+                    for (int o = 0; o < 8; o++)
+                        if (((o >> a) & 1) == up) mask |= (uint8_t)(1u << o);
+                    for (int i = 0; i < n[a]; i++) {
+                        uint8_t& v = out[(up ? n[a] - 1 - i : i) * step[a] + j * step[b] + k * step[d]];
+                        v |= m;
+                        m = v & mask;
+                    }
+                }
+    }
+    return s;
+}
+
 // Uploads one built slot into G (metadata into m); device allocations are recorded in allocs.
 static int uploadGrid(vrestir_handle* h, Grid& G, HostGrid& m, HostGrid& hg, std::vector<void*>& allocs) {
     std::memset(&G, 0, sizeof(Grid));
@@ -431,6 +461,10 @@ static int uploadGrid(vrestir_handle* h, Grid& G, HostGrid& m, HostGrid& hg, std
     G.occ = (const uint32_t*)p;
     G.occWords = (int32_t)(hg.occ.size() / 2);
     G.numBricks = hg.numBricks;
+    std::vector<uint8_t> ahead;
+    G.aheadShift = aheadTable(hg.brickTable, hg.nbx, hg.nby, hg.nbz, ahead);
+    if ((rc = up(ahead.data(), ahead.size(), &p))) return rc;
+    G.ahead = (const uint8_t*)p;
     if ((rc = up(hg.bounds.data(), hg.bounds.size() * 4, &p))) return rc;
     G.bounds = (const float*)p;
     if (hg.fp16) { if ((rc = up(hg.pool16.data(), hg.pool16.size() * 2, &p))) return rc; }
@@ -609,8 +643,10 @@ static int buildFrameDevice(vrestir_handle* h, hipStream_t st, const vrestir_vol
         DevBuf* b = f.built[slots[i].id];
         if ((rc = ck(growBuf(b[kBufTable], g.cells * 4, (void**)&g.table), "brick table")) ||
             (rc = ck(growBuf(b[kBufNodes], g.blocks * 4, (void**)&g.nodes), "block table")) ||
-            (rc = ck(growBuf(b[kBufWords], (g.cells + 31) / 32 * 8, (void**)&g.words), "occupancy words")))
+            (rc = ck(growBuf(b[kBufWords], (g.cells + 31) / 32 * 8, (void**)&g.words), "occupancy words")) ||
+            (rc = ck(growBuf(b[kBufAhead], kAheadBytes, (void**)&g.ahead), "ahead table")))
             return done(rc);
+        g.aheadShift = aheadShiftFor(g.nx / 8, g.ny / 8, g.nz / 8);
     }
     const int levels = std::min(d.numMips, 4) - 1;
     float* out[2][4] = {};
@@ -1484,6 +1520,7 @@ static int splitEnsure(vrestir_handle* h, int cap, size_t n) {
 static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
     a.splitTK = 0;
     a.splitMode = 0;
+    a.traceFlat = 0;
     if (!h->splitReuse) return VRESTIR_OK;
     const vrestir_params& p = h->P;
     const size_t n = (size_t)h->W * h->H;
@@ -1544,6 +1581,18 @@ static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
         (void)hipGetLastError();
         h->err.clear();
         return VRESTIR_OK;
+    }
+    if (tk == 2) {
+        // kTraceMarch: one grid and one filter for every ray, bricks, blocks within its LDS
+        // mask, and byte offsets into the pool within 32 bits. Shadow rays of TraceRays are
+        // all lighting rays
+        const Options& o = stage == VRESTIR_STAGE_TRACE_RAYS ? h->frame.initialOpt : h->frame.spatialOpt;
+        const bool one = stage == VRESTIR_STAGE_TRACE_RAYS ||
+                         (o.visibilityMipLevel == o.lightingMipLevel &&
+                          o.visibilityUseLinearSampler == o.lightingUseLinearSampler);
+        const Grid& g = h->sceneHost.grid[o.lightingMipLevel];
+        a.traceFlat = one && g.valid && g.numBricks > 0 && (size_t)g.nnx * g.nny * g.nnz <= kMarchBlocks &&
+                      (uint64_t)g.numBricks * kBrickVals * (g.fp16 ? 2u : 4u) <= 0xffffffffull;
     }
     a.split = h->split;
     a.split.cap = cap;
@@ -2239,8 +2288,7 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
         L.n = n;
         L.per = b->per;
         b->ops[k] = sp.op;
-        key.push_back(sp.op);
-        if (sp.op < 0) continue;
+        if (sp.op < 0) { key.push_back(sp.op); continue; }
         for (int i = 0; i < n; i++) {
             vrestir_handle* h = b->passes[i];
             LaunchArgs& a = b->argsHost[(size_t)k * kMaxBatch + i];
@@ -2257,6 +2305,8 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
             if (needSplit && (a.splitTK != wantTK || a.splitMode != 2))
                 return bfail(b, VRESTIR_EUNSUPPORTED, std::string("pass ") + std::to_string(i) +
                                                          ": a stage of this pass does not run in its split form");
+            if (sp.op == kOpSegmentsMarch && i == 0) b->ops[k] = kOpMarchFlat;
+            if (sp.op == kOpSegmentsMarch && !a.traceFlat) b->ops[k] = kOpSegmentsMarch;
             const bool seg = sp.op == kOpSegmentsMarch || sp.op == kOpSegmentsCells;
             const int W = a.width, H = a.height;
             const int gx = seg ? (W * H + 255) / 256 : (W + 15) / 16;
@@ -2268,6 +2318,7 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
             key.push_back(a.occBytes);
             key.push_back(tiles);
         }
+        key.push_back(b->ops[k]);
         if (sp.stage == VRESTIR_STAGE_SPATIAL_REUSE && sp.op == kOpSpatialReplay)
             for (int i = 0; i < n; i++) b->passes[i]->totalRoundId++;
     }
@@ -2300,7 +2351,7 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
                 }
                 continue;
             }
-            if (op == kOpSegmentsMarch || op == kOpSegmentsCells)
+            if (op == kOpSegmentsMarch || op == kOpMarchFlat || op == kOpSegmentsCells)
                 BHIP(b, launchBatchedSegments(b->stream, op, args, b->listsDev + k, b->countersDev + k, b->grid,
                                               b->occ[k]));
             else

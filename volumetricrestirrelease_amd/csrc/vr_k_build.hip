@@ -15,7 +15,7 @@
 // value of every brick of every level), the full-resolution clamped and dilated
 // grids are never stored (the fills of their occupied bricks form those values again),
 // the tables of all slots come from four launches together, and one wait for the
-// brick counts serves them all. 1024^3 with temperature, 4 mips, fp16: 31.6 -> 5.4 ms
+// brick counts serves them all. 1024^3 with temperature, 4 mips, fp16: 31.6 -> 5.35 ms
 // against a pass per step and a wait per slot (kLevels 2.5 ms, of which reading the grid
 // once takes 0.7, the temperature's kBrickMax 0.74 = 5.8 TB/s, the fills 1.7: their
 // VALU work per value); 96^3, 3 mips: 1.72 -> 0.15 ms.
@@ -323,34 +323,30 @@ struct TableJobs {
     BuildGrid g[kFrameSlots];
     BuildStats* stats;
 };
-__global__ __launch_bounds__(kBuildThreads) void kGridMax(const TableJobs J) {
-    const BuildGrid& g = J.g[blockIdx.y];
+// Each step is a body over a range of threads (i of n), so that a frame of small grids can
+// run all of them in one workgroup a slot (kTablesSmall) and a large one a launch each.
+__device__ __forceinline__ float gridMaxBody(const BuildGrid& g, size_t i, size_t n) {
     float m = 0.f;
-    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < g.cells; c += (size_t)gridDim.x * blockDim.x)
-        m = fmaxf(m, __uint_as_float(g.brickMax[c]));
-    m = laneMax(m, 1, 32);
-    if ((threadIdx.x & 63) == 0) maxInto(&J.stats->maxBits[blockIdx.y], m);
+    for (size_t c = i; c < g.cells; c += n) m = fmaxf(m, __uint_as_float(g.brickMax[c]));
+    return laneMax(m, 1, 32);
 }
 // Occupancy: does a brick hold a value that its stored form keeps above 0? Storing is
-// monotone, so its largest value tells. Also clears the block table.
-__global__ __launch_bounds__(kBuildThreads) void kWords(const TableJobs J, int fp16) {
-    const BuildGrid& g = J.g[blockIdx.y];
-    const float gmax = __uint_as_float(J.stats->maxBits[blockIdx.y]);
-    const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
-    for (size_t i = i0; i < g.blocks; i += stride) g.nodes[i] = 0u;
+// monotone, so its largest value tells. Also clears the block and ahead tables.
+__device__ __forceinline__ void wordsBody(const BuildGrid& g, float gmax, int fp16, size_t i, size_t n) {
+    for (size_t k = i; k < g.blocks; k += n) g.nodes[k] = 0u;
+    for (size_t k = i; k < kAheadBytes / 4; k += n) reinterpret_cast<uint32_t*>(g.ahead)[k] = 0u;
     // whole waves iterate together: 64 cells are two words
-    for (size_t c = i0; c - (threadIdx.x & 63) < g.cells; c += stride) {
+    for (size_t c = i; c - (threadIdx.x & 63) < g.cells; c += n) {
         const bool occ = c < g.cells && stored(__uint_as_float(g.brickMax[c]), gmax, fp16) > 0.f;
         const uint64_t bits = __ballot(occ);
         const int l = threadIdx.x & 63;
         if ((l & 31) == 0 && c < g.cells) g.words[2 * (c / 32)] = (uint32_t)(l ? bits >> 32 : bits);
     }
 }
-// Exclusive prefix of the words' popcounts into their second entries, one workgroup a
-// slot: 4096 consecutive words an iteration, scanned by wave and then across the waves.
-__global__ __launch_bounds__(1024) void kScanWords(const TableJobs J) {
-    const BuildGrid& g = J.g[blockIdx.y];
-    __shared__ uint32_t waveSum[16];
+// Exclusive prefix of the words' popcounts into their second entries, one workgroup of
+// 1024 a slot: 4096 consecutive words an iteration, scanned by wave and then across the
+// waves. Returns the number of bricks.
+__device__ __forceinline__ uint32_t scanBody(const BuildGrid& g, uint32_t* waveSum) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const size_t nw = (g.cells + 31) / 32;
     uint32_t base = 0u;
@@ -383,12 +379,12 @@ __global__ __launch_bounds__(1024) void kScanWords(const TableJobs J) {
         base = all;
         __syncthreads();
     }
-    if (threadIdx.x == 0) J.stats->count[blockIdx.y] = base;
+    return base;
 }
-__global__ __launch_bounds__(kBuildThreads) void kBrickIds(const TableJobs J) {
-    const BuildGrid& g = J.g[blockIdx.y];
+__device__ __forceinline__ void brickIdsBody(const BuildGrid& g, size_t i, size_t n) {
     const uint32_t nbx = g.nx / 8, nby = g.ny / 8;
-    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < g.cells; c += (size_t)gridDim.x * blockDim.x) {
+    const int as = g.aheadShift;
+    for (size_t c = i; c < g.cells; c += n) {
         const uint32_t bits = g.words[2 * (c / 32)], b = (uint32_t)(c % 32);
         if (!((bits >> b) & 1u)) { g.table[c] = kEmpty; continue; }
         const uint32_t id = g.words[2 * (c / 32) + 1] + (uint32_t)__popc(bits & ((1u << b) - 1u));
@@ -396,7 +392,88 @@ __global__ __launch_bounds__(kBuildThreads) void kBrickIds(const TableJobs J) {
         g.cellOf[id] = (uint32_t)c;
         const uint32_t r = (uint32_t)c / nbx, bx = (uint32_t)c % nbx, by = r % nby, bz = r / nby;
         g.nodes[(bx / 16) + (size_t)g.nnx * ((by / 16) + (size_t)g.nny * (bz / 16))] = 1u;
+        g.ahead[(bx >> as) + (((nbx - 1) >> as) + 1) * ((by >> as) + (((nby - 1) >> as) + 1) * (bz >> as))] = 0xFFu;
     }
+}
+// The ahead table (Grid::ahead) from the groups that brickIdsBody marked: per axis, the
+// octants that increase on it gather from the high side, the others from the low side; a
+// thread a line.
+__device__ __forceinline__ void aheadBody(const BuildGrid& g, uint8_t* t) {
+    const int n[3] = {((g.nx / 8 - 1) >> g.aheadShift) + 1, ((g.ny / 8 - 1) >> g.aheadShift) + 1,
+                      ((g.nz / 8 - 1) >> g.aheadShift) + 1};
+    const int all = n[0] * n[1] * n[2], step[3] = {1, n[0], n[0] * n[1]};
+    for (int i = threadIdx.x; i < all; i += blockDim.x) t[i] = g.ahead[i];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        __syncthreads();
+        const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+        const uint32_t up = a == 0 ? 0xAAu : (a == 1 ? 0xCCu : 0xF0u);
+        const int line = threadIdx.x;
+        if (line < n[b] * n[c]) {
+            uint8_t* l = t + (line % n[b]) * step[b] + (line / n[b]) * step[c];
+            uint32_t v[kAheadSide], m = 0u;
+#pragma unroll
+            for (int i = 0; i < kAheadSide; i++) v[i] = i < n[a] ? l[i * step[a]] : 0u;
+#pragma unroll
+            for (int i = kAheadSide - 1; i >= 0; i--) m = (v[i] |= m) & up;
+            m = 0u;
+#pragma unroll
+            for (int i = 0; i < kAheadSide; i++) m = (v[i] |= m) & ~up;
+#pragma unroll
+            for (int i = 0; i < kAheadSide; i++)
+                if (i < n[a]) l[i * step[a]] = (uint8_t)v[i];
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < all; i += blockDim.x) g.ahead[i] = t[i];
+}
+
+__global__ __launch_bounds__(kBuildThreads) void kGridMax(const TableJobs J) {
+    const float m = gridMaxBody(J.g[blockIdx.y], (size_t)blockIdx.x * blockDim.x + threadIdx.x,
+                                (size_t)gridDim.x * blockDim.x);
+    if ((threadIdx.x & 63) == 0) maxInto(&J.stats->maxBits[blockIdx.y], m);
+}
+__global__ __launch_bounds__(kBuildThreads) void kWords(const TableJobs J, int fp16) {
+    wordsBody(J.g[blockIdx.y], __uint_as_float(J.stats->maxBits[blockIdx.y]), fp16,
+              (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
+}
+__global__ __launch_bounds__(1024) void kScanWords(const TableJobs J) {
+    __shared__ uint32_t waveSum[16];
+    const uint32_t n = scanBody(J.g[blockIdx.y], waveSum);
+    if (threadIdx.x == 0) J.stats->count[blockIdx.y] = n;
+}
+__global__ __launch_bounds__(kBuildThreads) void kBrickIds(const TableJobs J) {
+    brickIdsBody(J.g[blockIdx.y], (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
+}
+__global__ __launch_bounds__(kAheadSide* kAheadSide) void kAhead(const TableJobs J) {
+    __shared__ uint8_t t[kAheadBytes];
+    aheadBody(J.g[blockIdx.y], t);
+}
+// All of it for a slot in one workgroup, for grids of at most kSmallCells bricks: five
+// launches' starts and gaps cost more than one workgroup's passes (a build of 96^3, 6
+// slots: 0.185 -> 0.152 ms; at 256^3 a pass is 32 iterations).
+constexpr size_t kSmallCells = 32768;
+__global__ __launch_bounds__(1024) void kTablesSmall(const TableJobs J, int fp16) {
+    const BuildGrid& g = J.g[blockIdx.y];
+    __shared__ uint32_t waveSum[16];
+    __shared__ float waveMax[16];
+    __shared__ uint8_t t[kAheadBytes];
+    const float m = gridMaxBody(g, threadIdx.x, 1024);
+    if ((threadIdx.x & 63) == 0) waveMax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    float gmax = 0.f;
+    for (int k = 0; k < 16; k++) gmax = fmaxf(gmax, waveMax[k]);
+    wordsBody(g, gmax, fp16, threadIdx.x, 1024);
+    __syncthreads();
+    const uint32_t n = scanBody(g, waveSum);
+    if (threadIdx.x == 0) {
+        J.stats->maxBits[blockIdx.y] = __float_as_uint(gmax);
+        J.stats->count[blockIdx.y] = n;
+    }
+    __syncthreads();
+    brickIdsBody(g, threadIdx.x, 1024);
+    __syncthreads();
+    aheadBody(g, t);
 }
 
 // Per brick its 10^3 apron values (stored form) and bounds {min, max, sum / 512, 0}.
@@ -561,11 +638,16 @@ hipError_t buildTables(hipStream_t st, const BuildGrid* grids, int n, bool fp16,
         J.g[i] = grids[i];
         cells = std::max(cells, grids[i].cells);
     }
+    if (cells <= kSmallCells) {
+        hipLaunchKernelGGL(kTablesSmall, dim3(1, n), dim3(1024), 0, st, J, fp16 ? 1 : 0);
+        return hipGetLastError();
+    }
     const dim3 g((unsigned)std::min<size_t>((cells + kBuildThreads - 1) / kBuildThreads, 512), n);
     hipLaunchKernelGGL(kGridMax, g, dim3(kBuildThreads), 0, st, J);
     hipLaunchKernelGGL(kWords, g, dim3(kBuildThreads), 0, st, J, fp16 ? 1 : 0);
     hipLaunchKernelGGL(kScanWords, dim3(1, n), dim3(1024), 0, st, J);
     hipLaunchKernelGGL(kBrickIds, g, dim3(kBuildThreads), 0, st, J);
+    hipLaunchKernelGGL(kAhead, dim3(1, n), dim3(kAheadSide * kAheadSide), 0, st, J);
     return hipGetLastError();
 }
 hipError_t buildFill(hipStream_t st, const BuildGrid* grids, const BuildStats& stats, int n, bool fp16) {
@@ -606,6 +688,8 @@ void buildDescribe(const BuildGrid& b, const BuildStats& stats, int i, bool fp16
     G.nodeTable = b.nodes;
     G.occ = b.words;
     G.occWords = (int32_t)((b.cells + 31) / 32);
+    G.ahead = b.ahead;
+    G.aheadShift = b.aheadShift;
     G.numBricks = stats.count[i];
     G.bounds = b.bounds;
     G.pool = b.pool;

@@ -102,9 +102,9 @@ static constexpr int kSegCap = 128;             // segment queue entries per wav
 static constexpr int kSegHigh = kSegCap - 64;   // the walk phase stops above this fill (<= 64 pushes per step)
 static constexpr int kWalkSteps = 32;           // walk-phase iterations before marching
 static constexpr int kNodeWords = 64;           // block-occupancy bits kept in LDS (2048 blocks)
-static constexpr int kRayRefill = 16;           // lanes that must want a ray before a refill round
+static constexpr int kRayRefill = 24;           // lanes that must want a ray before a refill round
 static constexpr int kCarryLanes = 32;          // march lanes left when the rest of the march is carried over
-static constexpr int kBlockBatch = 16;          // lanes at a block border before their block entries run
+static constexpr int kBlockBatch = 8;           // lanes at a block border before their block entries run
 static constexpr int kCellsPerStep = 1;         // empty cells a walking lane may cross per walk iteration
 
 struct SegQueue {
@@ -193,90 +193,6 @@ VR_DEV float footprintValue(const Footprint<FP16, LIN>& fp) {
     }
 }
 
-// Drains the wave's segment queue when every segment uses grid Gu with storage
-// format FP16 and filter LIN, software-pipelined: each iteration a lane fetches
-// the footprint of its segment's next sample (TrMarch's brick loop: up to 128
-// samples while inside the brick and before tFar) and steps past it, then adds
-// the sample it fetched the iteration before to its running sum, so a sample's
-// loads are in flight across a whole iteration. A lane whose segment has no next
-// sample takes the next segment of the queue in the same iteration. Samples of
-// one ray slot that follow each other in a lane add up in order; the sum goes to
-// the slot with an LDS float atomic when the lane moves to another slot.
-template <int FP16, int LIN>
-VR_DEV void marchPipelined(const Scene& S, const Grid& Gu, SegQueue& Q, int nSeg, uint64_t below) {
-    const gptr<char> pool = gbl<char>(Gu.pool);
-    const float dScale = S.densityScale, sigT = S.sigma_t;
-    int mHead = 0;  // wave-uniform
-    // issue side: the segment whose next sample is fetched
-    bool iHas = false;
-    int iOwner = 0, iIt = 0;
-    uint32_t iBrick = 0;
-    float iT = 0.f, iTStep = 0.f, iTFar = 0.f;
-    v3 iQ = V3(0.f), iDq = V3(0.f);
-    // the sample fetched in the previous iteration (its footprint alternates
-    // between fpA and fpB, so a fetch never waits to be copied)
-    bool fHas = false;
-    int fOwner = 0;
-    float fStep = 0.f;
-    Footprint<FP16, LIN> fpA{}, fpB{};
-    // compute side: the running sum of ray slot cOwner
-    int cOwner = -1;
-    float part = 0.f;
-    // one iteration: fetch the next sample into nxt, add the one in cur; false when all is done
-    auto iteration = [&](const Footprint<FP16, LIN>& cur, Footprint<FP16, LIN>& nxt) -> bool {
-        if (iHas && !(iIt < 128 && inBrick(iQ) && iT < iTFar)) iHas = false;
-        const uint64_t nm = __ballot(!iHas);
-        if (nm && mHead < nSeg) {
-            if (!iHas) {
-                const int e = mHead + __popcll(nm & below);
-                if (e < nSeg) {
-                    const int ow = Q.owner[e];
-                    iOwner = ow & 255;
-                    iIt = ow >> 8;
-                    iBrick = Q.brick[e];
-                    iT = Q.t[e];
-                    iQ = V3(Q.q[0][e], Q.q[1][e], Q.q[2][e]);
-                    iDq = V3(Q.dq[0][iOwner], Q.dq[1][iOwner], Q.dq[2][iOwner]);
-                    iTStep = Q.tStep[iOwner];
-                    iTFar = Q.tFar[iOwner];
-                    // a segment without a sample adds nothing
-                    iHas = iIt < 128 && inBrick(iQ) && iT < iTFar;
-                }
-            }
-            mHead += __popcll(nm);
-        }
-        // fetch the issue side's next sample and step past it
-        const bool nHas = iHas;
-        const int nOwner = iOwner;
-        const float nStep = iTStep;
-        fetchInside<FP16, LIN>(pool, iHas, iBrick, iQ, nxt);
-        if (iHas) {
-            iQ = iQ + iDq;
-            iT += 1.f * iTStep;
-            iIt++;
-        }
-        // add the sample fetched last iteration; its value is formed in every lane (from
-        // stale registers where nothing was fetched) so that the wait for cur's loads is
-        // not inside a branch: after it no path leaves a load pending on cur's registers
-        const float st = footprintValue<FP16, LIN>(cur) * dScale * sigT;
-        if (fHas && fOwner != cOwner) {
-            if (cOwner >= 0) atomicAdd(&Q.sum[cOwner], part);
-            cOwner = fOwner;
-            part = 0.f;
-        }
-        part = fHas ? part + -st * 1.f * fStep : part;
-        fHas = nHas;
-        fOwner = nOwner;
-        fStep = nStep;
-        return __ballot(fHas || iHas) != 0ull || mHead < nSeg;
-    };
-    for (;;) {
-        if (!iteration(fpA, fpB)) break;
-        if (!iteration(fpB, fpA)) break;
-    }
-    if (cOwner >= 0) atomicAdd(&Q.sum[cOwner], part);
-}
-
 // Drains the wave's segment queue: each lane marches a segment (TrMarch's brick
 // loop: up to 128 samples while inside the brick and before tFar) and takes the
 // next one as soon as it is done; the segment's sum goes to its ray's slot.
@@ -358,7 +274,6 @@ struct CellQueue {
     float sum[kRaySlots];
     float pos[3][kRaySlots], dir[3][kRaySlots];  // the index-space ray (vertex-shifted when trilinear)
     float tFar[kRaySlots];
-    int pend[kRaySlots];                         // unused: the analytic march carries nothing over
     int owner[kSegCap];                          // ray slot
     uint32_t brick[kSegCap];
     float tx[kSegCap];
@@ -483,6 +398,17 @@ VR_DEV bool segBlockEntry(const FlatWalk& w) { return w.blockEntry; }
 VR_DEV void segEnterBlock(Walker<2>&, const WalkCtx&) {}
 VR_DEV void segEnterBlock(FlatWalk& w, const WalkCtx& c) { w.enterBlock(c.g, c.nb); }
 
+// Ray r of a wave's 64 pixels: the pixel is the first whose inclusive ray count incl
+// exceeds r (cnt: the lane's own count). Every lane must take part.
+struct RayPick { int r, pixel, index; };
+VR_DEV RayPick pickRay(int r, int incl, int cnt) {
+    int lo = 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        if (__shfl(incl, lo + o - 1) <= r) lo += o;
+    return {r, lo, r - __shfl(incl - cnt, lo)};
+}
+
 // TK = 2: ray marching (SegQueue, brick-sample march); TK = 1: analytic tracking
 // (CellQueue, cell integration; launched only on a grid whose block bits fit LDS,
 // one grid and one filter for both ray kinds).
@@ -492,7 +418,6 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
                               float* __restrict__ trs, int cap, int numPixels, int blockX) {
     const Scene& S = *sc;
     occCacheLoad(S, fr.occSlot[0], fr.occSlot[1]);
-    __shared__ int pre[4][65];
     using Queue = std::conditional_t<TK == 2, SegQueue, CellQueue>;
     __shared__ Queue queues[4];
     __shared__ uint32_t nodeBits[kNodeWords];
@@ -506,25 +431,20 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
         const int y = __shfl_up(incl, o);
         if (lane >= o) incl += y;
     }
-    pre[wv][lane + 1] = incl;
-    if (lane == 0) pre[wv][0] = 0;
-    __syncthreads();
-    const int total = pre[wv][64];
+    const int total = __builtin_amdgcn_readlane(incl, 63);
     Queue& Q = queues[wv];
 
     const int vs = opt.visibilityMipLevel, ls = isFinal ? 0 : opt.lightingMipLevel;
     const bool oneSlot = vs == ls;
     const bool uniformLinear = opt.visibilityUseLinearSampler != 0;
-    // one grid, format and filter for every segment; the grid has bricks and byte offsets
-    // into its pool fit 32 bits
-    const bool uniformMarch = oneSlot && uniformLinear == (opt.lightingUseLinearSampler != 0) &&
-                              S.grid[vs].numBricks > 0 &&
-                              (uint64_t)S.grid[vs].numBricks * kBrickVals * (S.grid[vs].fp16 ? 2u : 4u) <=
-                                  0xffffffffull;
     // the walk grid's block occupancy as bits in LDS, when it fits
     const Grid& Gw = S.grid[vs];
     const int nNodes = Gw.nnx * Gw.nny * Gw.nnz;
     const bool nodeLds = oneSlot && nNodes <= kNodeWords * 32;
+    // the analytic walk's ahead table: with it the queue still leaves room for five
+    // workgroups per CU (five waves per SIMD at 96 VGPRs)
+    __shared__ uint32_t aheadBits[TK == 1 ? kAheadBytes / 4 : 1];
+    if constexpr (TK == 1) aheadLoad(Gw, aheadBits);
     if (nodeLds) {
         for (int i = threadIdx.x; i < kNodeWords; i += blockDim.x) {
             uint32_t bits = 0;
@@ -540,15 +460,17 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
     // with the block bits in LDS the walk iterates over bricks only (FlatWalk)
     const bool flat = nodeLds;
     WalkCtx wc{&S, vs, oneSlot, nb, {}, TK == 1};
-    if (flat) wc.g.init(S.grid[vs], vs);
+    if (flat) wc.g.init(S.grid[vs], vs, TK == 1 ? aheadBits : nullptr);
     auto trace = [&](auto& w) {
         w.active = false;
         int bank = 0;      // the current ray's slot is 2 * lane + bank
         int waitMask = 0;  // bit b: slot 2 * lane + b holds a walked ray awaiting its march
         int head = 0;      // next ray of the wave's queue (wave-uniform)
         int nSeg = 0;      // segments in the queue (wave-uniform)
-        Q.pend[2 * lane] = 0;
-        Q.pend[2 * lane + 1] = 0;
+        if constexpr (TK == 2) {
+            Q.pend[2 * lane] = 0;
+            Q.pend[2 * lane + 1] = 0;
+        }
         for (;;) {
             // ---- walk phase
             for (int step = 0; step < kWalkSteps && nSeg <= kSegHigh; step++) {
@@ -557,16 +479,11 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
                 // refill in rounds of at least kRayRefill lanes (or when no walk is left), so the
                 // wave waits for record loads less often
                 if (wm && (__popcll(wm) >= kRayRefill || !__ballot(w.active))) {
+                    const RayPick pick = pickRay(head + __popcll(wm & below), incl, cnt);
                     if (want) {
-                        const int r = head + __popcll(wm & below);
-                        if (r < total) {
-                            int lo = 0, hi = 64;  // the pixel q with pre[q] <= r < pre[q + 1]
-                            while (hi - lo > 1) {
-                                const int mid = (lo + hi) >> 1;
-                                if (pre[wv][mid] <= r) lo = mid; else hi = mid;
-                            }
-                            const int rec = (p0 + lo) * cap + (r - pre[wv][lo]);
-                            const int tri = (r - pre[wv][lo]) * numPixels + p0 + lo;
+                        if (pick.r < total) {
+                            const int rec = (p0 + pick.pixel) * cap + pick.index;
+                            const int tri = pick.index * numPixels + p0 + pick.pixel;
                             const TraceRec R = recs[rec];
                             const int kind = R.kind;
                             const int slot = kind == 0 ? vs : ls;
@@ -638,16 +555,6 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
                 if (uniformLinear) marchCells<true>(S, S.grid[vs], Q, nSeg, below);
                 else marchCells<false>(S, S.grid[vs], Q, nSeg, below);
                 nSeg = 0;
-            } else if (uniformMarch) {
-                const Grid& G = S.grid[vs];
-                if (G.fp16) {
-                    if (uniformLinear) marchPipelined<1, 1>(S, G, Q, nSeg, below);
-                    else marchPipelined<1, 0>(S, G, Q, nSeg, below);
-                } else {
-                    if (uniformLinear) marchPipelined<0, 1>(S, G, Q, nSeg, below);
-                    else marchPipelined<0, 0>(S, G, Q, nSeg, below);
-                }
-                nSeg = 0;
             } else {
                 const bool mayCarry = head < total || __ballot(w.active) != 0ull;
                 nSeg = marchPhase(S, Q, nSeg, below, mayCarry);
@@ -657,11 +564,13 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
 #pragma unroll
             for (int b = 0; b < 2; b++) {
                 const int rs = 2 * lane + b;
-                if (((waitMask >> b) & 1) && !Q.pend[rs]) {
+                bool pending = false;
+                if constexpr (TK == 2) pending = Q.pend[rs] != 0;
+                if (((waitMask >> b) & 1) && !pending) {
                     trs[Q.rec[rs]] = expf(Q.sum[rs]);
                     waitMask &= ~(1 << b);
                 }
-                Q.pend[rs] = 0;
+                if constexpr (TK == 2) Q.pend[rs] = 0;
             }
             waveSync();
             if (head >= total && !__ballot(w.active) && !__ballot(waitMask != 0)) break;
@@ -677,16 +586,300 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
         trace(w);
     }
 }
+// Five waves per SIMD (96 VGPRs, 32 KB of LDS): the cell walks' loads are dependent.
 template <int TK>
-__global__ __launch_bounds__(256) void kTraceSegments(const Scene* __restrict__ sc, const Frame fr, Options opt,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TK == 1 ? 5 : 4, 8)))
+void kTraceSegments(const Scene* __restrict__ sc, const Frame fr, Options opt,
                                                       int isFinal, const TraceRec* __restrict__ recs,
                                                       const int* __restrict__ counts, float* __restrict__ trs,
                                                       int cap, int numPixels) {
     traceSegmentsBody<TK>(sc, fr, opt, isFinal, recs, counts, trs, cap, numPixels, (int)blockIdx.x);
 }
 
+// ------------------------------------------------------------------ the march of one grid
+// The segment trace when every ray walks one grid with one filter (spatial, temporal and
+// shadow rays under the default options), the grid has at most kMarchBlocks blocks and its pool
+// is below 4 GiB: the launch checks all three. Rays are walked and refilled as above;
+// the queue keeps only what its march needs, so that four workgroups fit a CU's LDS
+// beside the occupancy and ahead tables. Bound by VALU issue (60 % of it at 45 of 64
+// lanes; the walk's steps 70 % of the instructions). 1080p, 512^3 cloud, the frame's four
+// traces: 17.2 ms as kTraceSegments handing whole segments to lanes, 13.4 with the
+// balanced march and the walk ended by the ahead table, 12.8 with 192 queue entries in
+// place of 128, refills of 24 lanes (16, 32: +1.5 %) and block entries of 8 (16: +1.5 %).
+// Five waves per SIMD (96 VGPRs, spilling): 17.3 ms.
+static constexpr int kMarchCap = 192;               // queue entries per wave
+static constexpr int kMarchHigh = kMarchCap - 64;
+struct MarchQueue {
+    int rec[kRaySlots];            // the ray's transmittance slot; sign bit: kind 1
+    float sum[kRaySlots];
+    float dq[3][kRaySlots];
+    uint32_t brick[kMarchCap];
+    float q[3][kMarchCap];
+    uint16_t owner[kMarchCap];     // ray slot | samples << 8
+    uint16_t first[64];            // per lane: its first segment | samples to skip in it << 8
+};
+struct MarchShared {
+    uint32_t ahead[kAheadBytes / 4];
+    uint32_t nodeBits[kMarchBlocks / 32];
+    MarchQueue q[4];
+};
+
+// Samples of the segment that starts at (t0, q0) in a brick the ray leaves at tExit:
+// TrMarch's brick loop takes up to 128 while inside the brick and before tFar. (The
+// first one of a block, whose walk starts at the offset entry, may lie before the
+// brick: such a segment has none.) Counted from the exit time; where rounding could
+// decide (t is rounded at every step of the loop), the loop itself is run without its
+// samples.
+VR_DEV int segmentSamples(float t0, v3 q0, v3 dq, float tStep, float invStep, float tExit, float tFar) {
+    if (!inBrick(q0)) return 0;
+    const float r = (fminf(tExit, tFar) - t0) * invStep;
+    const float tol = 1e-5f * (fabsf(t0) * invStep + 16.f);
+    if (tol < 0.25f && fabsf(r - rintf(r)) > tol && r < 127.f) return max((int)ceilf(r), 0);
+    int n = 0;
+    while (n < 128 && inBrick(q0) && t0 < tFar) {
+        q0 = q0 + dq;
+        t0 += tStep;
+        n++;
+    }
+    return n;
+}
+
+// Drains the wave's segment queue when every segment uses grid Gu with storage
+// format FP16 and filter LIN. The segments' sample counts are known, so the samples
+// of the whole queue, laid end to end, are dealt to the 64 lanes in equal runs: every
+// lane takes the same number of samples and crosses from one segment to the next
+// without looking at other lanes. (Handing whole segments to idle lanes left 24 of 64
+// lanes idle at the queues' tails and paid a ballot and a range test per sample.)
+// A lane's loads are in flight for an iteration: the footprint of the next sample is
+// fetched, alternating between two register sets, before the current one is used.
+// Sums are of the interpolated values; the completed ray scales them.
+template <int FP16, int LIN>
+VR_DEV void marchBalanced(const Grid& Gu, MarchQueue& Q, int nSeg) {
+    const gptr<char> pool = gbl<char>(Gu.pool);
+    const int lane = threadIdx.x & 63;
+    // first sample of each segment in the laid-out order, kPerLane segments a lane
+    constexpr int kPerLane = kMarchCap / 64;
+    const int e0 = kPerLane * lane;
+    int n[kPerLane], mine = 0;
+#pragma unroll
+    for (int k = 0; k < kPerLane; k++) {
+        n[k] = e0 + k < nSeg ? Q.owner[e0 + k] >> 8 : 0;
+        mine += n[k];
+    }
+    int incl = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+    }
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    const int per = (total + 63) >> 6;  // samples a lane
+    if (per == 0) return;
+    // the segment each lane starts in: a segment names the lanes whose run begins inside it
+    {
+        int s = incl - mine;
+        const float inv = 1.f / (float)per;
+#pragma unroll
+        for (int k = 0; k < kPerLane; k++) {
+            int l = (int)((float)s * inv);  // within one of s / per
+            l = max(l - 1, 0);
+            while (l * per < s) l++;
+            for (; l < 64 && l * per < s + n[k]; l++) Q.first[l] = (uint16_t)((e0 + k) | (l * per - s) << 8);
+            s += n[k];
+        }
+    }
+    waveSync();
+    int left = min(per, total - lane * per);  // samples this lane still fetches (<= 0: none)
+    const int f = left > 0 ? Q.first[lane] : 0;
+    int e = f & 255;
+    int rem = 0, owner = 0;  // samples left in the segment, its ray slot
+    uint32_t brick = 0;
+    v3 q = V3(0.f), dq = V3(0.f);
+    auto take = [&](int skip) {
+        const int ow = Q.owner[e];
+        owner = ow & 255;
+        rem = (ow >> 8) - skip;
+        brick = Q.brick[e];
+        dq = V3(Q.dq[0][owner], Q.dq[1][owner], Q.dq[2][owner]);
+        q = V3(Q.q[0][e], Q.q[1][e], Q.q[2][e]) + (float)skip * dq;
+        e++;
+    };
+    if (left > 0) take(f >> 8);
+    // the fetched sample: its ray slot, or -1; bit 8: the last of its run in that slot
+    int fOwner = -1;
+    float part = 0.f;
+    Footprint<FP16, LIN> fpA{}, fpB{};
+    auto iteration = [&](const Footprint<FP16, LIN>& cur, Footprint<FP16, LIN>& nxt) {
+        const bool has = left > 0;
+        fetchInside<FP16, LIN>(pool, has, brick, q, nxt);
+        int nOwner = -1;
+        if (has) {
+            q = q + dq;
+            rem--;
+            left--;
+            nOwner = owner | (rem == 0 || left == 0 ? 256 : 0);
+            if (rem == 0 && left > 0) take(0);
+        }
+        // the sample fetched last iteration; its value is formed in every lane so that the
+        // wait for its loads is not inside a branch
+        const float v = footprintValue<FP16, LIN>(cur);
+        part += fOwner >= 0 ? v : 0.f;
+        if (fOwner >= 256) {
+            atomicAdd(&Q.sum[fOwner & 255], part);
+            part = 0.f;
+        }
+        fOwner = nOwner;
+    };
+    // per fetches and one more use
+    for (int i = 0; i <= per; i += 2) {
+        iteration(fpA, fpB);
+        iteration(fpB, fpA);
+    }
+}
+
+VR_DEV void marchBody(MarchShared& sh, const Scene* __restrict__ sc, const Frame& fr, const Options& opt,
+                      const TraceRec* __restrict__ recs, const int* __restrict__ counts, float* __restrict__ trs,
+                      int cap, int numPixels, int blockX) {
+    const Scene& S = *sc;
+    occCacheLoad(S, fr.occSlot[0], fr.occSlot[1]);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int p0 = (blockX * 4 + wv) * 64;
+    const int cnt = p0 + lane < numPixels ? counts[p0 + lane] : 0;
+    int incl = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+    }
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    MarchQueue& Q = sh.q[wv];
+    const int slot = opt.visibilityMipLevel;
+    const Grid& G = S.grid[slot];
+    const int nNodes = G.nnx * G.nny * G.nnz;
+    for (int i = threadIdx.x; i * 32 < nNodes; i += blockDim.x) {
+        uint32_t bits = 0;
+        for (int b = 0; b < 32; b++) {
+            const int n = i * 32 + b;
+            if (n < nNodes && gbl<uint32_t>(G.nodeTable)[n] != 0u) bits |= 1u << b;
+        }
+        sh.nodeBits[i] = bits;
+    }
+    aheadLoad(G, sh.ahead);
+    __syncthreads();
+    FlatGrid g;
+    g.init(G, slot, sh.ahead);
+    const float scale = S.densityScale * S.sigma_t;
+    FlatWalk w;
+    w.active = false;
+    int bank = 0;      // the current ray's slot is 2 * lane + bank
+    int waitMask = 0;  // bit b: slot 2 * lane + b holds a walked ray awaiting its march
+    int head = 0;      // next ray of the wave's queue (wave-uniform)
+    int nSeg = 0;      // segments in the queue (wave-uniform)
+    for (;;) {
+        // ---- walk phase
+        for (int step = 0; step < kWalkSteps && nSeg <= kMarchHigh; step++) {
+            const bool want = !w.active && !((waitMask >> bank) & 1) && head < total;
+            const uint64_t wm = __ballot(want);
+            if (wm && (__popcll(wm) >= kRayRefill || !__ballot(w.active))) {
+                const RayPick pick = pickRay(head + __popcll(wm & below), incl, cnt);
+                if (want && pick.r < total) {
+                    const int tri = pick.index * numPixels + p0 + pick.pixel;
+                    const TraceRec R = recs[(size_t)(p0 + pick.pixel) * cap + pick.index];
+                    w.begin(S, G, slot, Ray{V3(R.ox, R.oy, R.oz), V3(R.dx, R.dy, R.dz), 0.f, R.tMax},
+                            R.kind == 0 ? opt.visibilityTStepScale : opt.lightingTStepScale, g, sh.nodeBits);
+                    if (w.active) {
+                        const int rs = 2 * lane + bank;
+                        Q.rec[rs] = tri | (R.kind == 0 ? 0 : (int)0x80000000u);
+                        Q.sum[rs] = 0.f;
+                        const v3 dq = 1.f * w.tStep * w.dda.dir;
+                        Q.dq[0][rs] = dq.x; Q.dq[1][rs] = dq.y; Q.dq[2][rs] = dq.z;
+                    } else {
+                        trs[tri] = 1.f;  // the ray meets no brick
+                    }
+                }
+                head += __popcll(wm);
+            }
+            if (!__ballot(w.active)) {
+                if (head >= total || !__ballot(!((waitMask >> bank) & 1))) break;
+                continue;
+            }
+            // block entries, batched: a lane at a block border waits until kBlockBatch lanes
+            // (or all walking lanes) are
+            const bool wasActive = w.active;
+            const uint64_t bm = __ballot(w.active && w.blockEntry);
+            if (bm && (__popcll(bm) >= kBlockBatch || bm == __ballot(w.active))) {
+                if (w.active && w.blockEntry) w.enterBlock(g, sh.nodeBits);
+            }
+            uint32_t bk = kEmpty;
+            float t0 = 0.f;
+            v3 q0 = V3(0.f);
+            int count = 0;
+            const int rs = 2 * lane + bank;
+            if (w.active && !w.blockEntry && w.step(g, bk, t0, q0))
+                count = segmentSamples(t0, q0, w.tStep * w.dda.dir, w.tStep, w.invStep, w.dda.ty, w.tFar);
+            if (wasActive && !w.active) {
+                waitMask |= 1 << bank;
+                bank ^= 1;
+            }
+            const uint64_t pm = __ballot(count > 0);
+            if (count > 0) {
+                const int e = nSeg + __popcll(pm & below);
+                Q.owner[e] = (uint16_t)(rs | count << 8);
+                Q.brick[e] = bk;
+                Q.q[0][e] = q0.x; Q.q[1][e] = q0.y; Q.q[2][e] = q0.z;
+            }
+            nSeg += __popcll(pm);
+        }
+        waveSync();
+        // ---- march phase
+        const bool lin = opt.visibilityUseLinearSampler != 0;
+        if (G.fp16) {
+            if (lin) marchBalanced<1, 1>(G, Q, nSeg);
+            else marchBalanced<1, 0>(G, Q, nSeg);
+        } else {
+            if (lin) marchBalanced<0, 1>(G, Q, nSeg);
+            else marchBalanced<0, 0>(G, Q, nSeg);
+        }
+        nSeg = 0;
+        waveSync();
+        // ---- rays whose walk ended are complete
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const int rs = 2 * lane + b;
+            if ((waitMask >> b) & 1) {
+                const int rec = Q.rec[rs];
+                const float tss = rec >= 0 ? opt.visibilityTStepScale : opt.lightingTStepScale;
+                trs[rec & 0x7FFFFFFF] = expf(-(Q.sum[rs] * scale) * FlatWalk::stepLength(S, slot, tss));
+            }
+        }
+        waitMask = 0;
+        waveSync();
+        if (head >= total && !__ballot(w.active)) break;
+    }
+}
+#ifndef VR_MARCH_WAVES
+#define VR_MARCH_WAVES 4
+#endif
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VR_MARCH_WAVES, 8)))
+void kTraceMarch(const Scene* __restrict__ sc, const Frame fr, Options opt,
+                                                   const TraceRec* __restrict__ recs, const int* __restrict__ counts,
+                                                   float* __restrict__ trs, int cap, int numPixels) {
+    __shared__ MarchShared sh;
+    marchBody(sh, sc, fr, opt, recs, counts, trs, cap, numPixels, (int)blockIdx.x);
+}
+
 hipError_t launchTraceSegments(const LaunchArgs& a, const Options& opt, bool isFinal) {
     const int n = a.width * a.height;
+    if (a.traceFlat) {
+        // the kernel walks and marches one grid with one filter; the plan says that it may
+        if (opt.visibilityMipLevel != opt.lightingMipLevel ||
+            opt.visibilityUseLinearSampler != opt.lightingUseLinearSampler)
+            return hipErrorInvalidValue;
+        hipLaunchKernelGGL(kTraceMarch, dim3((n + 255) / 256), dim3(256), a.occBytes, a.stream, a.scene, a.frame, opt,
+                           a.split.recs, a.split.counts, a.split.trs, a.split.cap, n);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(kTraceSegments<2>, dim3((n + 255) / 256), dim3(256), a.occBytes, a.stream, a.scene, a.frame,
                        opt, isFinal ? 1 : 0, a.split.recs, a.split.counts, a.split.trs, a.split.cap, n);
     return hipGetLastError();
@@ -724,11 +917,37 @@ VR_TRACING_KERNEL void kBatchedSegments(const LaunchArgs* __restrict__ args,
     }
 }
 
+// kTraceMarch over a batch's items (every instance's step is flat)
+VR_TRACING_KERNEL void kBatchedMarch(const LaunchArgs* __restrict__ args, const BatchList* __restrict__ list,
+                                     int* __restrict__ counter) {
+    __shared__ MarchShared sh;
+    __shared__ int sItem;
+    const int n = list->n, total = list->start[n], per = list->per;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) sItem = atomicAdd(counter, 1);
+        __syncthreads();
+        const int item = __builtin_amdgcn_readfirstlane(sItem);
+        if (item >= total) break;
+        int i = 0;
+        while (i + 1 < n && item >= list->start[i + 1]) i++;
+        const LaunchArgs& a = args[i];
+        const int t0 = (item - list->start[i]) * per, t1 = min(t0 + per, list->tiles[i]);
+        for (int t = t0; t < t1; t++) {
+            if (t > t0) __syncthreads();
+            marchBody(sh, a.scene, a.frame, a.frame.spatialOpt, a.split.recs, a.split.counts, a.split.trs, a.split.cap,
+                      a.width * a.height, t);
+        }
+    }
+}
+
 hipError_t launchBatchedSegments(hipStream_t st, int op, const LaunchArgs* args, const BatchList* list, int* counter,
                                  int grid, int occBytes) {
     if (grid <= 0) return hipErrorInvalidValue;
     if (op == kOpSegmentsMarch)
         hipLaunchKernelGGL(kBatchedSegments<2>, dim3(grid), dim3(256), occBytes, st, args, list, counter);
+    else if (op == kOpMarchFlat)
+        hipLaunchKernelGGL(kBatchedMarch, dim3(grid), dim3(256), occBytes, st, args, list, counter);
     else if (op == kOpSegmentsCells)
         hipLaunchKernelGGL(kBatchedSegments<1>, dim3(grid), dim3(256), occBytes, st, args, list, counter);
     else

@@ -19,6 +19,7 @@ struct LaunchArgs {
     int splitTK;   // > 0: run the reuse stage as record / trace / replay with tracker kind splitTK
     int splitMode; // the trace of that split: 1 = walker queue (kTraceQueue), 2 = brick segments (kTraceSegments)
     SplitBufs split;
+    int traceFlat; // the marched trace of that split runs as kTraceMarch (one grid, one filter, blocks in LDS)
     int64_t traceGridBlocks;  // 128^3 blocks of the grid the analytic cell trace walks (host-side count)
     const Scene* scene;
     Frame frame;
@@ -50,6 +51,7 @@ hipError_t launchReferenceLattice(const LaunchArgs& a, int stride, int spp, uint
 hipError_t launchTemporalReuse(const LaunchArgs& a);
 hipError_t launchSpatialReuse(const LaunchArgs& a);
 hipError_t launchFinalShading(const LaunchArgs& a);
+constexpr int kMarchBlocks = 2048;  // 128^3 blocks of a grid that kTraceMarch walks
 // Balanced trace of the rays recorded in a.split (vr_k_queue.hip); tk: 2 ray marching, 1 analytic.
 hipError_t launchTraceQueue(const LaunchArgs& a, const Options& opt, bool isFinal, int tk);
 hipError_t launchTraceSegments(const LaunchArgs& a, const Options& opt, bool isFinal);
@@ -72,7 +74,7 @@ struct BatchList {
 enum BatchOp {
     kOpFeatures = 0, kOpTrace, kOpTemporalRecord, kOpTemporalReplay, kOpCopyFeatures, kOpSpatialRecord,
     kOpSpatialReplay, kOpCopyReservoirs, kOpFinalRecord, kOpFinalReplay, kOpSegmentsMarch, kOpSegmentsCells,
-    kOpTraceLearned, kOpTemporalDirect, kOpProfile, kOpCount
+    kOpTraceLearned, kOpTemporalDirect, kOpProfile, kOpMarchFlat, kOpCount
 };
 // One persistent launch of `grid` workgroups draining the step's work list
 // (counter: the step's queue head, zero before the launch). args and list are
@@ -123,6 +125,8 @@ struct BuildGrid {
     unsigned* brickMax;             // scratch: the largest value per cell, as float bits
     uint32_t* cellOf;               // scratch: the cell of each brick
     uint32_t *table, *nodes, *words;
+    uint8_t* ahead;                 // Grid::ahead, kAheadBytes
+    int aheadShift;
     float* bounds;
     void* pool;
 };
@@ -145,7 +149,7 @@ hipError_t buildTables(hipStream_t st, const BuildGrid* grids, int n, bool fp16,
 hipError_t buildFill(hipStream_t st, const BuildGrid* grids, const BuildStats& stats, int n, bool fp16);
 void buildDescribe(const BuildGrid& b, const BuildStats& stats, int i, bool fp16, Grid& G);
 // A slot's device buffers, kept from one build to the next.
-enum { kBufTable = 0, kBufNodes, kBufWords, kBufBounds, kBufPool, kBufKinds };
+enum { kBufTable = 0, kBufNodes, kBufWords, kBufAhead, kBufBounds, kBufPool, kBufKinds };
 // Importance mip chain of a lat-long map: level k of dim >> k texels at imp + off[k].
 hipError_t launchEnvImportance(hipStream_t st, const float* tex, int W, int H, float* imp, const int* off, int dim,
                                int spp);

@@ -49,7 +49,21 @@ struct Grid {
     // number of occupied bricks in all earlier words: brick ids are assigned in
     // table order, so id = prefix + popcount(word bits below the brick's bit).
     const uint32_t* occ;          // occWords pairs {word, prefix}
+    // Where a walk can stop: per group of (1 << aheadShift)^3 brick cells, bit o set when
+    // an occupied brick lies in the group or ahead of it for a ray of octant o (bit 0 of
+    // o: x does not decrease, bits 1 and 2: y, z). At most kAheadSide groups a side, x
+    // fastest; nullptr: not known.
+    const uint8_t* ahead;
+    int32_t aheadShift;
+    int32_t pad2_;
 };
+static const int kAheadSide = 16;
+static const int kAheadBytes = kAheadSide * kAheadSide * kAheadSide;
+inline int aheadShiftFor(int nbx, int nby, int nbz) {
+    int s = 0;
+    while (((nbx - 1) >> s) >= kAheadSide || ((nby - 1) >> s) >= kAheadSide || ((nbz - 1) >> s) >= kAheadSide) s++;
+    return s;
+}
 
 struct Scene {
     Grid grid[kMaxSlots];

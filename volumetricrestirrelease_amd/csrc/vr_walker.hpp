@@ -286,19 +286,47 @@ struct Walker {
 // hierarchical walk's; over empty blocks the block-level side distances
 // accumulate as there.
 
+// ------------------------------------------------------------------ where a walk can stop
+// A ray leaves a sparse volume long before it leaves its grid: on a 512^3 cloud 7 of a
+// shadow or bounce ray's 12 brick steps cross nothing but empty cells behind the last
+// brick. A DDA only ever moves to higher (or lower) cells on an axis, so an empty cell
+// whose group has no occupied brick in or ahead of it for the ray's octant
+// (Grid::ahead) ends the walk: what is left of it has nothing to march. Only the walks
+// that keep the table in LDS ask; in the one-kernel traversals (`traverse`) the test
+// cost as much as it saved (TraceRays' record 5.4 -> 5.6 ms, path tracing 2 % slower).
+VR_DEV int rayOctant(v3 d) { return (d.x >= 0 ? 1 : 0) | (d.y >= 0 ? 2 : 0) | (d.z >= 0 ? 4 : 0); }
+VR_DEV int aheadIndex(int nbx, int nby, int s, int x, int y, int z) {
+    return (x >> s) + (((nbx - 1) >> s) + 1) * ((y >> s) + (((nby - 1) >> s) + 1) * (z >> s));
+}
+// A grid's ahead table into LDS (all bits set when it has none); a barrier must follow.
+VR_DEV void aheadLoad(const Grid& G, uint32_t* lds) {
+    gptr<uint32_t> a = gbl<uint32_t>(G.ahead);
+    for (int i = threadIdx.x; i < kAheadBytes / 4; i += blockDim.x) lds[i] = G.ahead ? a[i] : 0xFFFFFFFFu;
+}
+
 // The walk grid's brick occupancy, with its sizes held in registers.
 struct FlatGrid {
     int nbx, nby, nbz, nnx, nny, nnz;
     uint32_t numBricks;
     const uint2* occ;  // the grid's LDS occupancy table (occCacheLoad), or null: read brickTable
     const uint32_t* brickTable;
-    VR_DEV void init(const Grid& G, int slot) {
+    const uint8_t* ahead;  // the grid's LDS ahead table (aheadLoad), or null
+    int aheadShift;
+    VR_DEV void init(const Grid& G, int slot, const uint32_t* aheadLds) {
         nbx = G.nbx; nby = G.nby; nbz = G.nbz;
         nnx = G.nnx; nny = G.nny; nnz = G.nnz;
         numBricks = G.numBricks;
         brickTable = G.brickTable;
         const int k = slot == sOccSlot[0] ? 0 : (slot == sOccSlot[1] ? 1 : -1);
         occ = k < 0 ? nullptr : sOccTab + sOccOff[k];
+        ahead = reinterpret_cast<const uint8_t*>(aheadLds);
+        aheadShift = G.aheadShift;
+    }
+    // no brick in or ahead of an empty cell's group for the octant
+    VR_DEV bool nothingAhead(int octant, int x, int y, int z) const {
+        if (!ahead || (unsigned)x >= (unsigned)nbx || (unsigned)y >= (unsigned)nby || (unsigned)z >= (unsigned)nbz)
+            return false;
+        return ((ahead[aheadIndex(nbx, nby, aheadShift, x, y, z)] >> octant) & 1u) == 0u;
     }
     // brickLookup's answer
     VR_DEV uint32_t lookup(int bx, int by, int bz) const {
@@ -318,9 +346,16 @@ struct FlatWalk {
     Dda dda;
     float tNear, tFar, tStep, invStep;
     float tBlock;      // exit distance of the current 128^3 block
+    int octant;        // of the direction (rayOctant)
     int iter;
     bool active;
     bool blockEntry;   // tx passed tBlock: enterBlock() runs before the next step
+    // The march step of a grid slot
+    VR_DEV static float stepLength(const Scene& S, int slot, float tStepScale) {
+        int eff = slot >= 19 ? slot - 19 : slot;
+        eff = eff >= 8 ? eff - 8 : eff;
+        return S.tStep * S.worldScaling * tStepScale * (float)(eff + 1);
+    }
     // Walker<TK>::begin for a walk of grid G (slot `slot`) and the entry of its first
     // block: vc (analytic tracking with the trilinear filter) shifts the ray by half
     // a voxel and takes the hierarchical walk's up to three block-level steps while
@@ -330,15 +365,14 @@ struct FlatWalk {
         const float eps = 0.01f;
         Ray ray{xformP(G.w2i, rWorld.o), xformV(G.w2i, rWorld.d), rWorld.tMin, rWorld.tMax};
         if (vc) ray.o = ray.o - 0.5f;
-        int eff = slot >= 19 ? slot - 19 : slot;
-        eff = eff >= 8 ? eff - 8 : eff;
-        tStep = S.tStep * S.worldScaling * tStepScale * (float)(eff + 1);
+        tStep = stepLength(S, slot, tStepScale);
         invStep = 1.f / tStep;
         if (!intersectBounds(G, ray, tNear, tFar, vc)) {
             active = false;
             return;
         }
         dda.setFromRay(ray.o, ray.d, tNear + eps);
+        octant = rayOctant(ray.d);
         iter = 0;
         active = true;
         blockEntry = false;
@@ -423,12 +457,20 @@ struct FlatWalk {
             if (t < dda.tx) t += tStep;
             t0 = t;
             q0 = at(Ray{dda.pos, dda.dir, 0.f, 0.f}, t) - bmin;
+        } else if (g.nothingAhead(octant, cx, cy, cz)) {
+            active = false;
+            return false;
         }
+        leaveCell();
+        return seg;
+    }
+    // Past the current cell; at a block border past tFar the walk is over (enterBlock)
+    VR_DEV void leaveCell() {
         dda.step();
-        dda.tx += eps;
+        dda.tx += 0.01f;
         iter++;
         blockEntry = dda.tx > tBlock;
-        return seg;
+        if (blockEntry && dda.tx > tFar) active = false;
     }
     // One brick cell of an analytic-tracking walk: true with the brick, the
     // distance tx its cell walk starts from and its brick coordinates when the
@@ -441,7 +483,6 @@ struct FlatWalk {
     // such a brick adds nothing and the tracker goes on to the next one, where
     // its first cell, already past tFar, adds the clamped term and ends it.
     VR_DEV bool stepCells(const FlatGrid& g, uint32_t& bk, float& txOut, i3v& cell) {
-        const float eps = 0.01f;
         if (!(iter < 4096)) {
             active = false;
             return false;
@@ -459,10 +500,11 @@ struct FlatWalk {
             const i3v lp = {(int)fl.x, (int)fl.y, (int)fl.z};
             last = (unsigned)lp.x < 8u && (unsigned)lp.y < 8u && (unsigned)lp.z < 8u;
         }
-        dda.step();
-        dda.tx += eps;
-        iter++;
-        blockEntry = dda.tx > tBlock;
+        if (!seg && g.nothingAhead(octant, cell.x, cell.y, cell.z)) {
+            active = false;
+            return false;
+        }
+        leaveCell();
         if (last) active = false;
         return seg;
     }
