@@ -1725,6 +1725,8 @@ static int stageArgs(vrestir_handle* h, hipStream_t st, int stage, int round, fl
     a.height = h->H;
     a.scene = h->sceneDev;
     a.frame = h->frame;
+    a.frame.traceShift = traceShift((int64_t)h->W * h->H);
+    a.frame.laneShift = h->inBatch ? 0 : stageShift((int64_t)h->W * h->H);
     a.offsets = h->offsetsDev;
     a.features = h->features;
     a.featuresT = h->featuresT;
@@ -2309,7 +2311,8 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
             if (sp.op == kOpSegmentsMarch && !a.traceFlat) b->ops[k] = kOpSegmentsMarch;
             const bool seg = sp.op == kOpSegmentsMarch || sp.op == kOpSegmentsCells;
             const int W = a.width, H = a.height;
-            const int gx = seg ? (W * H + 255) / 256 : (W + 15) / 16;
+            const int per = 4 * (64 >> a.frame.traceShift);  // pixels a workgroup of a trace
+            const int gx = seg ? (W * H + per - 1) / per : (W + 15) / 16;
             const int tiles = seg ? gx : gx * ((H + 15) / 16);
             L.gx[i] = gx;
             L.tiles[i] = tiles;

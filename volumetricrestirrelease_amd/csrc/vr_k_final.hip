@@ -4,7 +4,7 @@
 namespace vr {
 
 hipError_t launchFinalShading(const LaunchArgs& a) {
-    const dim3 g = tiles(a.width, a.height), blk(256, 1, 1);
+    const dim3 g = tiles(a.frame), blk(256, 1, 1);
     const Options& fo = a.frame.finalOpt;
     const bool fiAnalytic = fo.visibilityTrackingMethod == 1u && fo.lightingTrackingMethod == 1u;
     if (a.splitTK == 1 && fiAnalytic) {

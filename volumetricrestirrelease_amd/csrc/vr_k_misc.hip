@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void kProfile(const Scene* __restrict__ sc, co
     profileBody(sc, fr, launchBlock());
 }
 hipError_t launchProfile(const LaunchArgs& a) {
-    hipLaunchKernelGGL(kProfile, tiles(a.width, a.height), dim3(256), a.occBytes, a.stream, a.scene, a.frame);
+    hipLaunchKernelGGL(kProfile, tiles(a.frame), dim3(256), a.occBytes, a.stream, a.scene, a.frame);
     return hipGetLastError();
 }
 
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void kTrack(const Scene* __restrict__ sc, cons
 
 
 hipError_t launchStage(const LaunchArgs& a) {
-    const dim3 g = tiles(a.width, a.height), blk(256, 1, 1);
+    const dim3 g = tiles(a.frame), blk(256, 1, 1);
     switch (a.stage) {
         case 0:
             hipLaunchKernelGGL(kFeatures, dim3(g.x, g.y, a.frame.prof.tau ? 2 : 1), blk, a.occBytes, a.stream, a.scene,

@@ -423,8 +423,8 @@ VR_DEV void traceSegmentsBody(const Scene* __restrict__ sc, const Frame& fr, con
     __shared__ uint32_t nodeBits[kNodeWords];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
-    const int p0 = (blockX * 4 + wv) * 64;
-    const int cnt = p0 + lane < numPixels ? counts[p0 + lane] : 0;
+    const int per = 64 >> fr.traceShift, p0 = (blockX * 4 + wv) * per;
+    const int cnt = lane < per && p0 + lane < numPixels ? counts[p0 + lane] : 0;
     int incl = cnt;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -744,8 +744,8 @@ VR_DEV void marchBody(MarchShared& sh, const Scene* __restrict__ sc, const Frame
     occCacheLoad(S, fr.occSlot[0], fr.occSlot[1]);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
-    const int p0 = (blockX * 4 + wv) * 64;
-    const int cnt = p0 + lane < numPixels ? counts[p0 + lane] : 0;
+    const int per = 64 >> fr.traceShift, p0 = (blockX * 4 + wv) * per;
+    const int cnt = lane < per && p0 + lane < numPixels ? counts[p0 + lane] : 0;
     int incl = cnt;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -869,6 +869,11 @@ void kTraceMarch(const Scene* __restrict__ sc, const Frame fr, Options opt,
     marchBody(sh, sc, fr, opt, recs, counts, trs, cap, numPixels, (int)blockIdx.x);
 }
 
+// workgroups of a trace: four waves of 64 >> traceShift pixels
+static dim3 traceGrid(const LaunchArgs& a) {
+    const int per = 4 * (64 >> a.frame.traceShift);
+    return dim3((a.width * a.height + per - 1) / per);
+}
 hipError_t launchTraceSegments(const LaunchArgs& a, const Options& opt, bool isFinal) {
     const int n = a.width * a.height;
     if (a.traceFlat) {
@@ -876,11 +881,11 @@ hipError_t launchTraceSegments(const LaunchArgs& a, const Options& opt, bool isF
         if (opt.visibilityMipLevel != opt.lightingMipLevel ||
             opt.visibilityUseLinearSampler != opt.lightingUseLinearSampler)
             return hipErrorInvalidValue;
-        hipLaunchKernelGGL(kTraceMarch, dim3((n + 255) / 256), dim3(256), a.occBytes, a.stream, a.scene, a.frame, opt,
+        hipLaunchKernelGGL(kTraceMarch, traceGrid(a), dim3(256), a.occBytes, a.stream, a.scene, a.frame, opt,
                            a.split.recs, a.split.counts, a.split.trs, a.split.cap, n);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(kTraceSegments<2>, dim3((n + 255) / 256), dim3(256), a.occBytes, a.stream, a.scene, a.frame,
+    hipLaunchKernelGGL(kTraceSegments<2>, traceGrid(a), dim3(256), a.occBytes, a.stream, a.scene, a.frame,
                        opt, isFinal ? 1 : 0, a.split.recs, a.split.counts, a.split.trs, a.split.cap, n);
     return hipGetLastError();
 }
@@ -962,7 +967,7 @@ hipError_t launchTraceCells(const LaunchArgs& a, const Options& opt, bool isFina
     if (opt.visibilityMipLevel != opt.lightingMipLevel || a.traceGridBlocks <= 0 ||
         a.traceGridBlocks > kNodeWords * 32)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(kTraceSegments<1>, dim3((n + 255) / 256), dim3(256), a.occBytes, a.stream, a.scene, a.frame,
+    hipLaunchKernelGGL(kTraceSegments<1>, traceGrid(a), dim3(256), a.occBytes, a.stream, a.scene, a.frame,
                        opt, isFinal ? 1 : 0, a.split.recs, a.split.counts, a.split.trs, a.split.cap, n);
     return hipGetLastError();
 }

@@ -4,7 +4,7 @@
 namespace vr {
 
 hipError_t launchTemporalReuse(const LaunchArgs& a) {
-    const dim3 g = tiles(a.width, a.height), blk(256, 1, 1);
+    const dim3 g = tiles(a.frame), blk(256, 1, 1);
     const Options& so = a.frame.spatialOpt;
     const bool spMarch = so.visibilityTrackingMethod == 2u && so.lightingTrackingMethod == 2u;
     if (a.splitTK == 2 && spMarch) {

@@ -13,12 +13,14 @@ namespace vr {
 template <int B>
 __global__ __launch_bounds__(256) void kReferenceLattice(const Scene* __restrict__ sc, const Frame fr, int stride,
                                                          int lw, int lh, int spp, uint32_t sn,
-                                                         float4* __restrict__ out) {
+                                                         int laneShift, float4* __restrict__ out) {
     const Scene& S = *sc;
     const Frame& F = fr;
     occCacheLoad(S, F.occSlot[0], F.occSlot[1]);
-    const int i = blockIdx.x * 16 + (threadIdx.x & 15), j = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (i >= lw || j >= lh) return;
+    // the first 64 >> laneShift lanes of each wave hold points, as in pixelOf
+    const int lane = threadIdx.x & 63, per = 64 >> laneShift, k = (threadIdx.x >> 6) * per + lane;
+    const int i = blockIdx.x * 16 + (k & 15), j = blockIdx.y * (16 >> laneShift) + (k >> 4);
+    if (lane >= per || i >= lw || j >= lh) return;
     const int x = stride * i + stride / 2, y = stride * j + stride / 2;
     Rng rng = rngCreate(x, y, sn + blockIdx.z);
     Ray ray{ld3(F.cam.pos), rayDir(F.cam, x, y, F.width, F.height), 0.f, kTMax};
@@ -37,9 +39,10 @@ hipError_t launchReferenceLattice(const LaunchArgs& a, int stride, int spp, uint
                                   float4* out) {
     int lw, lh;
     latticeSize(a.width, a.height, stride, lw, lh);
-    const dim3 g((lw + 15) / 16, (lh + 15) / 16, chunks), blk(256, 1, 1);
+    const int ls = latticeShift((int64_t)lw * lh * chunks), rows = 16 >> ls;
+    const dim3 g((lw + 15) / 16, (lh + rows - 1) / rows, chunks), blk(256, 1, 1);
     VR_DISPATCH_B(a, hipLaunchKernelGGL(kReferenceLattice<B>, g, blk, a.occBytes, a.stream, a.scene, a.frame, stride,
-                                        lw, lh, spp, sampleNumber, out))
+                                        lw, lh, spp, sampleNumber, ls, out))
     return hipGetLastError();
 }
 
@@ -48,7 +51,7 @@ hipError_t launchReferenceLattice(const LaunchArgs& a, int stride, int spp, uint
 // replay the candidates with their transmittances, then run the pixels the replay
 // could not finish (a transmittance of exactly 0) in one kernel.
 static hipError_t launchTraceRaysSplit(const LaunchArgs& a, bool spMarch) {
-    const dim3 g = tiles(a.width, a.height), blk(256, 1, 1);
+    const dim3 g = tiles(a.frame), blk(256, 1, 1);
     hipError_t e = launchZeroCounters(a.stream, a.split.fix, 1);
     if (e != hipSuccess) return e;
     VR_DISPATCH_B(a, hipLaunchKernelGGL((kTraceSplit<B, 2, 2, kRecord>), g, blk, a.occBytes, a.stream, a.scene,
@@ -84,7 +87,7 @@ static hipError_t launchTraceRaysSplit(const LaunchArgs& a, bool spMarch) {
 }
 
 hipError_t launchTraceRays(const LaunchArgs& a) {
-    const dim3 g = tiles(a.width, a.height), blk(256, 1, 1);
+    const dim3 g = tiles(a.frame), blk(256, 1, 1);
     const Options& so = a.frame.spatialOpt;
     const bool spMarch = so.visibilityTrackingMethod == 2u && so.lightingTrackingMethod == 2u;
     const bool inMarch = a.frame.initialOpt.lightingTrackingMethod == 2u;

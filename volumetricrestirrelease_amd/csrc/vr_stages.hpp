@@ -24,9 +24,11 @@ VR_DEV VBlock launchBlock() { return {(int)blockIdx.x, (int)blockIdx.y}; }
 struct PixelIdx { int x, y, id; bool ok; };
 VR_DEV PixelIdx pixelOf(const Frame& F, VBlock b) {
     PixelIdx p;
-    p.x = b.x * 16 + (threadIdx.x & 15);
-    p.y = b.y * 16 + (threadIdx.x >> 4);
-    p.ok = p.x < F.width && p.y < F.height;
+    // the first 64 >> laneShift lanes of each wave hold the pixels of a 16-wide tile
+    const int lane = threadIdx.x & 63, per = 64 >> F.laneShift, i = (threadIdx.x >> 6) * per + lane;
+    p.x = b.x * 16 + (i & 15);
+    p.y = b.y * (16 >> F.laneShift) + (i >> 4);
+    p.ok = lane < per && p.x < F.width && p.y < F.height;
     p.id = p.y * F.width + p.x;
     return p;
 }
@@ -43,7 +45,10 @@ VR_DEV bool inRange(int x, int y, int W, int H) { return x >= 0 && x < W && y >=
 #endif
 #define VR_TRACE_KERNEL __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VR_TRACE_WAVES, 8)))
 
-static inline dim3 tiles(int W, int H) { return dim3((W + 15) / 16, (H + 15) / 16, 1); }
+static inline dim3 tiles(const Frame& F) {
+    const int h = 16 >> F.laneShift;
+    return dim3((F.width + 15) / 16, (F.height + h - 1) / h, 1);
+}
 
 // Expands `body` with a compile-time B for the four supported path lengths.
 #define VR_DISPATCH_B(a, body)                                   \

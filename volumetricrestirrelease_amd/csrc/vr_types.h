@@ -201,6 +201,8 @@ struct Frame {
     int32_t outputMotionVec;
     int32_t useSurfaceScene;      // GenerateFeatures intersects the triangles and writes the V-buffer
     int32_t occSlot[2];           // grid slots whose occupancy tables the kernel keeps in LDS (-1: none)
+    int32_t laneShift;            // pixels a wave of a stage kernel: 64 >> laneShift (stageShift; 0 in batches)
+    int32_t traceShift;           // the same for the waves of the segment traces (traceShift)
     CameraFrame cam, prevCam;
     float prevView[16], prevProj[16];
     EnvXf env[2];                 // environment orientation: [0] this frame, [1] the previous frame
@@ -209,6 +211,28 @@ struct Frame {
     Options initialOpt, spatialOpt, finalOpt;
     CamProfile prof;
 };
+// How thinly a launch over n pixels is spread: a wave takes 64 >> shift of them. A wave
+// runs as long as the longest of its lanes' walks, one divergent path after another, so a
+// launch too small to fill the chip many times over finishes sooner with fewer pixels a
+// wave and more waves, up to `waves` of them. Four waves of the tracing kernels reside on
+// each of 1024 SIMDs. Measured (frame, us; one wave a 64 pixels first):
+//   stage kernels: 4096 waves, 4 pixels at least: 96x64 957 -> 748 together with the
+//     traces; 2048: 480x270 +5 %, 8192: 640x360 +6 %;
+//   segment traces (a wave keeps its 64 lanes busy from its pixels' rays, so more waves
+//     only cost their set-up): 16384, one pixel at least: 640x360 1607 -> 1280, 400x225
+//     2743 (4096 waves) -> 2150; 8192: 640x360 1361, 32768: 1337, 480x270 +3 %;
+//   path-traced lattices (lanes that end leave the wave idle): 8192: 240x135 points x 4
+//     14.1 -> 12.3 ms; 4096: 13.4.
+// Sums of a ray's optical depth depend on the segment traces' spread (their order), so a
+// batch gives each of its passes the spread it has alone.
+inline int laneShiftFor(int64_t n, int64_t waves, int most) {
+    int s = 0;
+    while (s < most && ((n << (s + 1)) + 63) / 64 <= waves) s++;
+    return s;
+}
+inline int stageShift(int64_t n) { return laneShiftFor(n, 4096, 4); }
+inline int traceShift(int64_t n) { return laneShiftFor(n, 16384, 6); }
+inline int latticeShift(int64_t n) { return laneShiftFor(n, 8192, 4); }
 // A transmittance ray recorded by the record pass of a reuse kernel
 // (world-space origin and direction, tMax, and which options trace it:
 // 0 = the visibility options, 1 = the lighting options).
