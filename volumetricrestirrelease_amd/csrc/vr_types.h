@@ -220,7 +220,9 @@ struct Frame {
 //     traces; 2048: 480x270 +5 %, 8192: 640x360 +6 %;
 //   segment traces (a wave keeps its 64 lanes busy from its pixels' rays, so more waves
 //     only cost their set-up): 16384, one pixel at least: 640x360 1607 -> 1280, 400x225
-//     2743 (4096 waves) -> 2150; 8192: 640x360 1361, 32768: 1337, 480x270 +3 %;
+//     2743 (4096 waves) -> 2150; 8192: 640x360 1361, 32768: 1337, 480x270 +3 %; and never
+//     more than 32 pixels: 1080p 28.2 -> 26.6 ms (16: 26.5), six views of 256^2 to 1440x810
+//     in a batch 24.6 -> 24.3 (with 65536 waves: 25.6);
 //   path-traced lattices (lanes that end leave the wave idle): 8192: 240x135 points x 4
 //     14.1 -> 12.3 ms; 4096: 13.4.
 // Sums of a ray's optical depth depend on the segment traces' spread (their order), so a
@@ -231,7 +233,10 @@ inline int laneShiftFor(int64_t n, int64_t waves, int most) {
     return s;
 }
 inline int stageShift(int64_t n) { return laneShiftFor(n, 4096, 4); }
-inline int traceShift(int64_t n) { return laneShiftFor(n, 16384, 6); }
+inline int traceShift(int64_t n) {
+    const int s = laneShiftFor(n, 16384, 6);
+    return s > 0 ? s : 1;
+}
 inline int latticeShift(int64_t n) { return laneShiftFor(n, 8192, 4); }
 // A transmittance ray recorded by the record pass of a reuse kernel
 // (world-space origin and direction, tMax, and which options trace it:
