@@ -50,8 +50,8 @@ HBM_PEAK_GBS = 8000.0
 # measured by this run: see the `traffic_source` field.
 PROFILE_TRAFFIC = {
     "file": "profiles/SpatialReuse_config1_1080p.md",
-    "bytes": {"SpatialReuse": 33.395e9, "TraceRays": 15.489e9, "FinalShading": 4.360e9, "TemporalReuse": 3.376e9,
-              "GenerateFeatures": 0.183e9, "CopyReservoirs": 0.156e9},
+    "bytes": {"SpatialReuse": 28.155e9, "TraceRays": 15.610e9, "FinalShading": 3.863e9, "TemporalReuse": 3.165e9,
+              "GenerateFeatures": 2.495e9, "CopyReservoirs": 0.156e9},
 }
 LATTICE = 8
 QUALITY_FRAMES = 60
