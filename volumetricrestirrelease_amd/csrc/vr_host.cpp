@@ -1602,7 +1602,7 @@ static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
 }
 
 // The camera-ray profiles of the open frame (profileTr in vr_pass.hpp): made when the
-// spatial visibility rays are ray-marched and the stages run in their split forms.
+// spatial rays are ray-marched and the stages run in their split forms.
 // A row has an entry per march step of the longest ray the grid can have (its
 // diagonal); rows that would not fit the budget or three quarters of the free memory
 // are not made, and the rays are traced where they are needed.
@@ -1611,8 +1611,9 @@ static void profilePlan(vrestir_handle* h, Frame& F) {
     F.prof = CamProfile{};
     const vrestir_params& p = h->P;
     const Options& so = F.spatialOpt;
-    if (h->splitReuse != 2 || so.visibilityTrackingMethod != 2u || p.useReference || p.useSurfaceScene || F.noReuse ||
-        h->freezeFrame)
+    // (the kernels of other tracker mixes trace every ray)
+    if (h->splitReuse != 2 || so.visibilityTrackingMethod != 2u || so.lightingTrackingMethod != 2u || p.useReference ||
+        p.useSurfaceScene || F.noReuse || h->freezeFrame)
         return;
     const Scene& S = h->sceneHost;
     const int slot = so.visibilityMipLevel;
