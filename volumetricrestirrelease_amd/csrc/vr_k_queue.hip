@@ -8,6 +8,7 @@
 // its 64 pixels. Idle lanes are refilled together once a quarter of the wave is
 // idle, so the set-up code runs at a useful width. The transmittance of each
 // ray is written at its record's index for the replay pass.
+#include "vr_segment.hpp"
 #include "vr_stages.hpp"
 #include "vr_walker.hpp"
 
@@ -624,24 +625,15 @@ struct MarchShared {
     MarchQueue q[4];
 };
 
-// Samples of the segment that starts at (t0, q0) in a brick the ray leaves at tExit:
-// TrMarch's brick loop takes up to 128 while inside the brick and before tFar. (The
-// first one of a block, whose walk starts at the offset entry, may lie before the
-// brick: such a segment has none.) Counted from the exit time; where rounding could
-// decide (t is rounded at every step of the loop), the loop itself is run without its
-// samples.
-VR_DEV int segmentSamples(float t0, v3 q0, v3 dq, float tStep, float invStep, float tExit, float tFar) {
-    if (!inBrick(q0)) return 0;
-    const float r = (fminf(tExit, tFar) - t0) * invStep;
-    const float tol = 1e-5f * (fabsf(t0) * invStep + 16.f);
-    if (tol < 0.25f && fabsf(r - rintf(r)) > tol && r < 127.f) return max((int)ceilf(r), 0);
-    int n = 0;
-    while (n < 128 && inBrick(q0) && t0 < tFar) {
-        q0 = q0 + dq;
-        t0 += tStep;
-        n++;
-    }
-    return n;
+// Samples of the segment at (t0, q0) of the brick that w just stepped out of: exactly the
+// march loop's count (vr_segment.hpp). None when the first one of a block, whose walk
+// starts at the offset entry, lies before the brick. (A bound on the rounding of the time
+// alone miscounted 5e-8 to 1e-6 of the segments, 80 to 250 pixels of a 1080p frame of a
+// 512^3 cloud; the certain count costs 0.8 % of that frame: 20.8 -> 21.0 ms.)
+VR_DEV int segmentSamples(const FlatWalk& w, float t0, v3 q0) {
+    const v3 dq = 1.f * w.tStep * w.dda.dir;
+    const float r = (fminf(w.dda.ty, w.tFar) - t0) * w.invStep;
+    return segmentCount(r, t0, q0.x, q0.y, q0.z, dq.x, dq.y, dq.z, w.tStep, w.tFar);
 }
 
 // Drains the wave's segment queue when every segment uses grid Gu with storage
@@ -817,7 +809,7 @@ VR_DEV void marchBody(MarchShared& sh, const Scene* __restrict__ sc, const Frame
             int count = 0;
             const int rs = 2 * lane + bank;
             if (w.active && !w.blockEntry && w.step(g, bk, t0, q0))
-                count = segmentSamples(t0, q0, w.tStep * w.dda.dir, w.tStep, w.invStep, w.dda.ty, w.tFar);
+                count = segmentSamples(w, t0, q0);
             if (wasActive && !w.active) {
                 waitMask |= 1 << bank;
                 bank ^= 1;
