@@ -446,8 +446,14 @@ int32_t vrestir_learned_train(vrestir_handle* h, void* stream, const float* recs
  * when the initial lighting rays use ray marching and the learned proposal is off.
  * A pixel whose resampling draws differ from the record's (a candidate weight that
  * its real shadow transmittance makes zero) is traced again in one kernel, so the
- * results agree with one kernel's to float rounding. 0 runs TraceRays as one kernel. */
-enum { VRESTIR_TUNE_SPLIT_REUSE = 1, VRESTIR_TUNE_SPLIT_TRACE = 2 };
+ * results agree with one kernel's to float rounding. 0 runs TraceRays as one kernel.
+ * VRESTIR_TUNE_PROFILE_MB (default VRESTIR_DEFAULT_PROFILE_MB; with
+ * VRESTIR_TUNE_SPLIT_REUSE 2): the most device memory, in MiB, that the handle's
+ * camera-ray profiles may take (one float per pixel and march step of the grid's
+ * diagonal). They are made only while half of the device's memory stays free beside
+ * them and the ray records; 0, or a frame that needs more, traces the rays instead. */
+enum { VRESTIR_TUNE_SPLIT_REUSE = 1, VRESTIR_TUNE_SPLIT_TRACE = 2, VRESTIR_TUNE_PROFILE_MB = 3 };
+#define VRESTIR_DEFAULT_PROFILE_MB 16384
 int32_t vrestir_set_tuning(vrestir_handle* h, int32_t key, int32_t value);
 
 /* ---- ground truth and error (AccumulatePass double mode, AccumulatePass.cpp:42,93;

@@ -32,6 +32,7 @@ BRICK_FP32, BRICK_FP16 = 0, 1
 
 TUNE_SPLIT_REUSE = 1
 TUNE_SPLIT_TRACE = 2
+TUNE_PROFILE_MB = 3
 
 STAGE_GENERATE_FEATURES, STAGE_TRACE_RAYS, STAGE_TEMPORAL_REUSE, STAGE_SPATIAL_REUSE, \
     STAGE_COPY_RESERVOIRS, STAGE_FINAL_SHADING = range(6)

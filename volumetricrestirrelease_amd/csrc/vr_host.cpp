@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -54,6 +55,9 @@ struct VolumeFrame {
     int numMips = 0;
     float tStep = 1.f, superVoxelDiag = 1.f;
 };
+
+// Camera-ray profiles are optional: by default at most 16 GiB a handle.
+static const size_t kProfileBudget = (size_t)VRESTIR_DEFAULT_PROFILE_MB << 20;
 
 struct vrestir_handle {
     int device = 0;
@@ -107,6 +111,9 @@ struct vrestir_handle {
     DevBuf profTau, profMeta;
     bool profReady = false;
     hipStream_t profStream = nullptr;
+    size_t profBudget = kProfileBudget;  // VRESTIR_TUNE_PROFILE_MB
+    size_t profRefused = 0;              // bytes the device had no room for (until options or size change)
+    bool reserving = false;              // a batch's reservation pass: records only, no profiles
     // textured environment map: texels, importance mip chain, orientation now and at the last frame
     float* envTexDev = nullptr;
     float* envImpDev = nullptr;
@@ -175,6 +182,14 @@ static void freeProfile(vrestir_handle* h) {
     freeBuf(h->profMeta);
     h->profReady = false;
 }
+// hipMalloc for what a frame cannot do without: the profiles give way to it.
+static hipError_t allocForFrame(vrestir_handle* h, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess || !h->profTau.p) return e;
+    (void)hipGetLastError();
+    freeProfile(h);
+    return hipMalloc(p, bytes);
+}
 static void freeSplit(vrestir_handle* h) {
     dfree(h->split.recs); dfree(h->split.trs); dfree(h->split.dens); dfree(h->split.counts); dfree(h->split.plan);
     dfree(h->split.fix);
@@ -183,6 +198,8 @@ static void freeSplit(vrestir_handle* h) {
 }
 static void freeFrameBuffers(vrestir_handle* h) {
     freeSplit(h);
+    freeProfile(h);
+    h->profRefused = 0;
     for (int i = 0; i < 2; i++) { dfree(h->res[i]); dfree(h->extra[i]); dfree(h->color[i]); }
     dfree(h->resT); dfree(h->extraT); dfree(h->features); dfree(h->featuresT); dfree(h->vbuf); dfree(h->outInternal);
     h->W = h->H = 0;
@@ -1185,14 +1202,14 @@ static int learnedFrameBuffers(vrestir_handle* h) {
     const size_t n = (size_t)h->W * h->H;
     if (h->lCdfPixels != n) {
         dfree(h->lCdf);
-        HIPCHK(h, hipMalloc((void**)&h->lCdf, n * 64));
+        HIPCHK(h, allocForFrame(h, (void**)&h->lCdf, n * 64));
         HIPCHK(h, hipMemset(h->lCdf, 0, n * 64));
         h->lCdfPixels = n;
     }
     const int slots = learnedSlots(h->W, h->H, h->L);
     if (h->lRecSlots != slots) {
         dfree(h->lRecs);
-        HIPCHK(h, hipMalloc((void**)&h->lRecs, (size_t)slots * kLearnedRecFloats * 4));
+        HIPCHK(h, allocForFrame(h, (void**)&h->lRecs, (size_t)slots * kLearnedRecFloats * 4));
         HIPCHK(h, hipMemset(h->lRecs, 0, (size_t)slots * kLearnedRecFloats * 4));
         h->lRecSlots = slots;
     }
@@ -1202,7 +1219,7 @@ static int learnedPartials(vrestir_handle* h, int records) {
     const int waves = (records + 31) / 32;
     if (waves > h->lPartialWaves) {
         dfree(h->lPartial);
-        HIPCHK(h, hipMalloc((void**)&h->lPartial, (size_t)waves * kLearnedPartialStride * 4));
+        HIPCHK(h, allocForFrame(h, (void**)&h->lPartial, (size_t)waves * kLearnedPartialStride * 4));
         h->lPartialWaves = waves;
     }
     return VRESTIR_OK;
@@ -1385,6 +1402,16 @@ extern "C" int32_t vrestir_learned_train(vrestir_handle* h, void* stream, const 
     return learnedStep(h, (hipStream_t)stream, recsDev, n);
 }
 
+// Whether the open frame's options use camera-ray profiles: the spatial rays are
+// ray-marched and the stages run in their split forms (the kernels of other tracker
+// mixes trace every ray and would not read them).
+static bool profileWanted(const vrestir_handle* h) {
+    const Frame& F = h->frame;
+    const Options& so = F.spatialOpt;
+    return h->splitReuse == 2 && h->profBudget > 0 && so.visibilityTrackingMethod == 2u &&
+           so.lightingTrackingMethod == 2u && !F.useReference && !F.useSurfaceScene && !F.noReuse && !h->freezeFrame;
+}
+
 // Frame set-up: reallocation, history reset on option change, round
 // bookkeeping and the three SamplingOptions (VR/VolumetricReSTIR.cpp:339-496).
 extern "C" int32_t vrestir_prepare_frame(vrestir_handle* h, int32_t W, int32_t H) {
@@ -1398,6 +1425,7 @@ extern "C" int32_t vrestir_prepare_frame(vrestir_handle* h, int32_t W, int32_t H
         h->frameCount = 0;
         h->temporalAccumulated = false;
         h->optionsChanged = false;
+        h->profRefused = 0;
     }
     if (W != h->W || H != h->H || p.maxBounces != h->allocB) {
         int rc = allocFrameBuffers(h, W, H, p.maxBounces);
@@ -1474,7 +1502,10 @@ extern "C" int32_t vrestir_prepare_frame(vrestir_handle* h, int32_t W, int32_t H
     if (learnedActive(h)) {
         int rc = learnedFrameBuffers(h);
         if (rc) return rc;
+        const int K = std::max(1, h->L.trainStepsPerFrame);
+        if (h->L.train && (rc = learnedPartials(h, (h->lRecSlots + K - 1) / K))) return rc;
     }
+    if (!profileWanted(h) && !h->freezeFrame) freeProfile(h);
     h->totalRoundId = 0;
     h->profReady = false;
     h->frameOpen = true;
@@ -1504,12 +1535,15 @@ static int occPlan(const vrestir_handle* h, int a, int b, int slots[2]) {
 // frame fit kSplitBudget; otherwise each runs in one kernel. The record buffers
 // hold the larger per-pixel capacity; each stage strides them by its own.
 static const size_t kSplitBudget = (size_t)48 << 30;
+static size_t splitBytes(size_t n, int cap) {
+    return n * (size_t)cap * (sizeof(TraceRec) + 2 * sizeof(float)) + n * 8;
+}
 static int splitEnsure(vrestir_handle* h, int cap, size_t n) {
     if (h->split.cap >= cap && h->splitPixels == n) return VRESTIR_OK;
     freeSplit(h);
-    HIPCHK(h, hipMalloc((void**)&h->split.recs, n * (size_t)cap * sizeof(TraceRec)));
-    HIPCHK(h, hipMalloc((void**)&h->split.trs, n * (size_t)cap * sizeof(float)));
-    HIPCHK(h, hipMalloc((void**)&h->split.dens, n * (size_t)cap * sizeof(float)));
+    HIPCHK(h, allocForFrame(h, (void**)&h->split.recs, n * (size_t)cap * sizeof(TraceRec)));
+    HIPCHK(h, allocForFrame(h, (void**)&h->split.trs, n * (size_t)cap * sizeof(float)));
+    HIPCHK(h, allocForFrame(h, (void**)&h->split.dens, n * (size_t)cap * sizeof(float)));
     HIPCHK(h, hipMalloc((void**)&h->split.counts, n * sizeof(int32_t)));
     HIPCHK(h, hipMalloc((void**)&h->split.plan, n * sizeof(uint32_t)));
     HIPCHK(h, hipMalloc((void**)&h->split.fix, sizeof(int32_t)));
@@ -1517,70 +1551,104 @@ static int splitEnsure(vrestir_handle* h, int cap, size_t n) {
     h->splitPixels = n;
     return VRESTIR_OK;
 }
-static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
-    a.splitTK = 0;
-    a.splitMode = 0;
-    a.traceFlat = 0;
-    if (!h->splitReuse) return VRESTIR_OK;
+// The ray slots per pixel of a stage's split under the open frame's options, and the
+// tracker kind of its rays; 0: the stage runs in one kernel.
+static int splitSlots(const vrestir_handle* h, int stage, int& tk) {
+    tk = 0;
+    if (!h->splitReuse) return 0;
     const vrestir_params& p = h->P;
-    const size_t n = (size_t)h->W * h->H;
-    int cap = 0, tk = 0;
     if (stage == VRESTIR_STAGE_TRACE_RAYS) {
         // the shadow rays of the candidates (ray marching only; not with the learned
         // proposal, the reference path tracer, or without reuse)
         const Frame& F = h->frame;
         if (h->splitReuse != 2 || !h->splitTrace || h->inBatch || learnedActive(h) || p.useReference || F.noReuse ||
             F.initialOpt.lightingTrackingMethod != 2u)
-            return VRESTIR_OK;
+            return 0;
         const int M = std::max(1, p.initialM), B = std::max(1, p.maxBounces);
-        cap = std::max(M * B, candStashSlots(M, B));  // one shadow ray per vertex; the free-flight samples
         tk = 2;
-    } else if (stage == VRESTIR_STAGE_SPATIAL_REUSE) {
+        return std::max(M * B, candStashSlots(M, B));  // one shadow ray per vertex; the free-flight samples
+    }
+    if (stage == VRESTIR_STAGE_SPATIAL_REUSE) {
         const Options& so = h->frame.spatialOpt;
-        if (so.visibilityTrackingMethod != 2u || so.lightingTrackingMethod != 2u) return VRESTIR_OK;
+        if (so.visibilityTrackingMethod != 2u || so.lightingTrackingMethod != 2u) return 0;
         const int K = p.spatialSampleCount;
         const int evals = p.spatialMISMethod == VRESTIR_MIS_TALBOT ? K * (K - 1) : K - 1;
-        cap = std::max(1, evals * (p.maxBounces + 1));
         tk = 2;
-    } else if (stage == VRESTIR_STAGE_TEMPORAL_REUSE) {
+        return std::max(1, evals * (p.maxBounces + 1));
+    }
+    if (stage == VRESTIR_STAGE_TEMPORAL_REUSE) {
         // the segment trace only; rays on the previous frame's grids (animated volumes) run in one kernel
         const Options& so = h->frame.spatialOpt;
         if (h->splitReuse != 2 || so.visibilityTrackingMethod != 2u || so.lightingTrackingMethod != 2u ||
             h->frame.prevGridOffset != 0)
-            return VRESTIR_OK;
-        cap = 2 * (p.maxBounces + 1);  // two target evaluations of b + 1 rays each
+            return 0;
         tk = 2;
-    } else if (stage == VRESTIR_STAGE_FINAL_SHADING) {
+        return 2 * (p.maxBounces + 1);  // two target evaluations of b + 1 rays each
+    }
+    if (stage == VRESTIR_STAGE_FINAL_SHADING) {
         const Options& fo = h->frame.finalOpt;
         if (fo.visibilityTrackingMethod != 1u || fo.lightingTrackingMethod != 1u || p.useReference ||
             h->frame.visualizeTransmittance)
-            return VRESTIR_OK;
+            return 0;
         // the analytic segment trace only (mode 2): one grid whose blocks fit its LDS bit mask, one filter
         const Grid& g0 = h->sceneHost.grid[fo.visibilityMipLevel];
         const bool uniformFilter = fo.visibilityUseLinearSampler == fo.lightingUseLinearSampler;
         if (h->splitReuse != 2 || fo.visibilityMipLevel != 0 || !g0.valid ||
             (size_t)g0.nnx * g0.nny * g0.nnz > 2048 || !uniformFilter)
-            return VRESTIR_OK;
-        cap = p.maxBounces + 1;  // the primary ray, one per extra bounce, the light ray
+            return 0;
         tk = 1;
-        a.traceGridBlocks = (int64_t)g0.nnx * g0.nny * g0.nnz;
-    } else {
-        return VRESTIR_OK;
+        return p.maxBounces + 1;  // the primary ray, one per extra bounce, the light ray
     }
-    // the record buffers must fit the budget and the device's free memory (keeping
-    // a quarter of it); a failed allocation falls back to the single kernel
-    const size_t need = n * (size_t)cap * (sizeof(TraceRec) + 2 * sizeof(float)) + n * 8;
-    const size_t held = h->splitPixels * (size_t)h->split.cap * (sizeof(TraceRec) + 2 * sizeof(float)) +
-                        h->splitPixels * 8;
+    return 0;
+}
+// Makes the record buffers hold cap slots a pixel: they must fit the budget and the
+// device's free memory (keeping a quarter of it), the profiles' counted with it, which
+// are given up where they stand in the way. false: the stage runs in one kernel.
+static bool splitReserve(vrestir_handle* h, int cap) {
+    const size_t n = (size_t)h->W * h->H;
+    if (h->split.cap >= cap && h->splitPixels == n) return true;
+    const size_t need = splitBytes(n, cap), held = h->splitPixels ? splitBytes(h->splitPixels, h->split.cap) : 0;
     size_t freeB = 0, totalB = 0;
-    if (need > kSplitBudget) return VRESTIR_OK;
-    if (need > held && hipMemGetInfo(&freeB, &totalB) == hipSuccess && need > (freeB + held) / 4 * 3)
-        return VRESTIR_OK;
+    if (need > kSplitBudget) return false;
+    if (need > held && hipMemGetInfo(&freeB, &totalB) == hipSuccess && need > (freeB + held) / 4 * 3) {
+        if (need > (freeB + held + h->profTau.cap + h->profMeta.cap) / 4 * 3) return false;
+        freeProfile(h);
+    }
     if (splitEnsure(h, cap, n) != VRESTIR_OK) {
         freeSplit(h);
         (void)hipGetLastError();
         h->err.clear();
-        return VRESTIR_OK;
+        return false;
+    }
+    return true;
+}
+// The records of every stage of the open frame, the largest that fit.
+static void splitReserveFrame(vrestir_handle* h) {
+    const vrestir_params& p = h->P;
+    std::vector<int> caps;
+    auto add = [&](int stage) {
+        int tk = 0;
+        const int cap = splitSlots(h, stage, tk);
+        if (cap > 0) caps.push_back(cap);
+    };
+    add(VRESTIR_STAGE_TRACE_RAYS);
+    if (p.enableTemporalReuse) add(VRESTIR_STAGE_TEMPORAL_REUSE);
+    if (p.enableSpatialReuse && p.spatialReuseRounds > 0) add(VRESTIR_STAGE_SPATIAL_REUSE);
+    add(VRESTIR_STAGE_FINAL_SHADING);
+    std::sort(caps.begin(), caps.end(), std::greater<int>());
+    for (int cap : caps)
+        if (splitReserve(h, cap)) return;
+}
+static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
+    a.splitTK = 0;
+    a.splitMode = 0;
+    a.traceFlat = 0;
+    int tk = 0;
+    const int cap = splitSlots(h, stage, tk);
+    if (cap == 0 || !splitReserve(h, cap)) return VRESTIR_OK;
+    if (tk == 1) {
+        const Grid& g0 = h->sceneHost.grid[h->frame.finalOpt.visibilityMipLevel];
+        a.traceGridBlocks = (int64_t)g0.nnx * g0.nny * g0.nnz;
     }
     if (tk == 2) {
         // kTraceMarch: one grid and one filter for every ray, bricks, blocks within its LDS
@@ -1601,24 +1669,15 @@ static int splitPlan(vrestir_handle* h, LaunchArgs& a, int stage) {
     return VRESTIR_OK;
 }
 
-// The camera-ray profiles of the open frame (profileTr in vr_pass.hpp): made when the
-// spatial rays are ray-marched and the stages run in their split forms.
-// A row has an entry per march step of the longest ray the grid can have (its
-// diagonal); rows that would not fit the budget or three quarters of the free memory
-// are not made, and the rays are traced where they are needed.
-static const size_t kProfileBudget = (size_t)16 << 30;
-static void profilePlan(vrestir_handle* h, Frame& F) {
-    F.prof = CamProfile{};
-    const vrestir_params& p = h->P;
-    const Options& so = F.spatialOpt;
-    // (the kernels of other tracker mixes trace every ray)
-    if (h->splitReuse != 2 || so.visibilityTrackingMethod != 2u || so.lightingTrackingMethod != 2u || p.useReference ||
-        p.useSurfaceScene || F.noReuse || h->freezeFrame)
-        return;
+// Entries of a camera-ray profile's row: one per march step of the longest ray the grid
+// can have (its diagonal); 0: the frame has no profiles.
+static size_t profileRow(const vrestir_handle* h) {
+    if (!profileWanted(h)) return 0;
+    const Options& so = h->frame.spatialOpt;
     const Scene& S = h->sceneHost;
     const int slot = so.visibilityMipLevel;
     const Grid& G = S.grid[slot];
-    if (!G.valid) return;
+    if (!G.valid) return 0;
     const double tStep = (double)S.tStep * S.worldScaling * so.visibilityTStepScale * (slot + 1);
     // world vectors of the box's edges: rows of the inverse of w2i's linear part, times its sizes
     const float* M = G.w2i;
@@ -1639,19 +1698,42 @@ static void profilePlan(vrestir_handle* h, Frame& F) {
         longest = std::max(longest, std::sqrt(l2));
     }
     const double steps = longest / tStep + 2.0;
-    if (!(steps > 0.0) || !(steps < 65000.0)) return;
-    const size_t n = (size_t)h->W * h->H, rowLen = (size_t)steps + 1;
+    return steps > 0.0 && steps < 65000.0 ? (size_t)steps + 1 : 0;
+}
+static size_t profileBytes(const vrestir_handle* h) {
+    return (size_t)h->W * h->H * profileRow(h) * sizeof(float);
+}
+// Whether the open frame's profiles are still to be allocated.
+static bool profileMissing(const vrestir_handle* h) {
+    const size_t need = profileBytes(h);
+    return need > h->profTau.cap && need <= h->profBudget && !(h->profRefused && need >= h->profRefused);
+}
+// The camera-ray profiles of the open frame (profileTr in vr_pass.hpp). They are
+// optional where the records are not (a stage without records runs in one kernel, a
+// batch not at all): the frame's records are reserved first, the rows must fit the
+// handle's budget and leave half of the device's memory free, and they are given back
+// when records need the room, or when the options or the frame's size change so that
+// they are not used. Without them the rays are traced where they are needed.
+static void profilePlan(vrestir_handle* h, Frame& F) {
+    F.prof = CamProfile{};
+    const size_t n = (size_t)h->W * h->H, rowLen = profileRow(h);
     const size_t need = n * rowLen * sizeof(float), meta = n * 2 * sizeof(float);
-    if (need > kProfileBudget) return;
-    if (need > h->profTau.cap) {
+    if (need == 0) return;
+    if (profileMissing(h)) {
         size_t freeB = 0, totalB = 0;
-        if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || need > (freeB + h->profTau.cap) / 4 * 3) return;
+        if (hipMemGetInfo(&freeB, &totalB) != hipSuccess || freeB + h->profTau.cap < need + totalB / 2)
+            h->profRefused = need;
+    }
+    if (need > h->profBudget || (need > h->profTau.cap && !profileMissing(h))) {
+        freeProfile(h);
+        return;
     }
     void *tau = nullptr, *mt = nullptr;
     const void* before = h->profTau.p;
     if (growBuf(h->profTau, need, &tau) != hipSuccess || growBuf(h->profMeta, meta, &mt) != hipSuccess) {
         (void)hipGetLastError();
         freeProfile(h);
+        h->profRefused = need;
         return;
     }
     if (tau != before) h->profReady = false;
@@ -1678,6 +1760,11 @@ extern "C" int32_t vrestir_set_tuning(vrestir_handle* h, int32_t key, int32_t va
         case VRESTIR_TUNE_SPLIT_TRACE:
             if (value < 0 || value > 1) return fail(h, VRESTIR_EINVAL, "split TraceRays must be 0 or 1");
             h->splitTrace = value;
+            return VRESTIR_OK;
+        case VRESTIR_TUNE_PROFILE_MB:
+            if (value < 0) return fail(h, VRESTIR_EINVAL, "the profile budget must not be negative");
+            h->profBudget = (size_t)value << 20;
+            h->profRefused = 0;
             return VRESTIR_OK;
         default: return fail(h, VRESTIR_EINVAL, "unknown tuning key");
     }
@@ -1780,14 +1867,18 @@ static int stageArgs(vrestir_handle* h, hipStream_t st, int stage, int round, fl
         case VRESTIR_STAGE_FINAL_SHADING: oa = F.finalOpt.visibilityMipLevel; ob = 0; break;
         default: break;
     }
-    if (stage != VRESTIR_STAGE_COPY_RESERVOIRS && stage != VRESTIR_STAGE_FINAL_SHADING) profilePlan(h, a.frame);
-    if (stage == VRESTIR_STAGE_GENERATE_FEATURES && !a.frame.prof.tau) ob = -1;
-    a.occBytes = occPlan(h, oa, ob, a.frame.occSlot);
+    const bool profiled = !h->reserving && stage != VRESTIR_STAGE_COPY_RESERVOIRS &&
+                          stage != VRESTIR_STAGE_FINAL_SHADING;
+    if (profiled && profileMissing(h)) splitReserveFrame(h);
     if (stage == VRESTIR_STAGE_TRACE_RAYS || stage == VRESTIR_STAGE_TEMPORAL_REUSE ||
         stage == VRESTIR_STAGE_SPATIAL_REUSE || stage == VRESTIR_STAGE_FINAL_SHADING) {
         int rc = splitPlan(h, a, stage);
         if (rc) return rc;
     }
+    // after the records: reserving them may give the profiles back
+    if (profiled) profilePlan(h, a.frame);
+    if (stage == VRESTIR_STAGE_GENERATE_FEATURES && !a.frame.prof.tau) ob = -1;
+    a.occBytes = occPlan(h, oa, ob, a.frame.occSlot);
     return VRESTIR_OK;
 }
 
@@ -2248,26 +2339,48 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
     // when it needs more rays per pixel than they hold, which would leave the
     // arguments of an earlier step of this frame pointing at freed buffers. Run
     // every step's plan once, so the buffers hold the frame's largest capacity,
-    // then build the arguments that are launched.
+    // then build the arguments that are launched. Profiles are planned with those, from
+    // the memory that every pass's records leave; where they hold memory from earlier
+    // frames that a pass's records need now, all are given back and the pass runs again.
     int temporalTK = -1;
-    {
+    for (int attempt = 0;; attempt++) {
         std::vector<int> rounds(n);
-        for (int i = 0; i < n; i++) rounds[i] = b->passes[i]->totalRoundId;
-        for (const Step& sp : steps) {
+        bool refused = false, held = false, mixed = false;
+        int rc = VRESTIR_OK;
+        temporalTK = -1;
+        for (int i = 0; i < n; i++) {
+            rounds[i] = b->passes[i]->totalRoundId;
+            b->passes[i]->reserving = true;
+        }
+        for (size_t k = 0; k < steps.size() && rc == VRESTIR_OK; k++) {
+            const Step& sp = steps[k];
             if (sp.op < 0) continue;
-            for (int i = 0; i < n; i++) {
+            for (int i = 0; i < n && rc == VRESTIR_OK; i++) {
+                vrestir_handle* h = b->passes[i];
                 LaunchArgs tmp;
-                int rc = stageArgs(b->passes[i], b->stream, sp.stage, sp.round, nullptr, tmp);
-                if (rc) return bfail(b, rc, std::string("pass ") + std::to_string(i) + ": " + b->passes[i]->err);
-                if (sp.op == kOpSpatialReplay) b->passes[i]->totalRoundId++;
+                rc = stageArgs(h, b->stream, sp.stage, sp.round, nullptr, tmp);
+                if (rc) { rc = bfail(b, rc, std::string("pass ") + std::to_string(i) + ": " + h->err); break; }
+                int tk = 0;
+                refused = refused || (splitSlots(h, sp.stage, tk) > 0 && tmp.splitTK == 0);
+                held = held || h->profTau.p;
+                if (sp.op == kOpSpatialReplay) h->totalRoundId++;
                 if (sp.op == kOpTemporalRecord) {
-                    if (temporalTK >= 0 && temporalTK != tmp.splitTK)
-                        return bfail(b, VRESTIR_EUNSUPPORTED, "passes differ in the form of their temporal reuse");
+                    mixed = mixed || (temporalTK >= 0 && temporalTK != tmp.splitTK);
                     temporalTK = tmp.splitTK;
                 }
             }
         }
-        for (int i = 0; i < n; i++) b->passes[i]->totalRoundId = rounds[i];
+        for (int i = 0; i < n; i++) {
+            b->passes[i]->totalRoundId = rounds[i];
+            b->passes[i]->reserving = false;
+        }
+        if (rc) return rc;
+        if (refused && held && attempt == 0) {
+            for (vrestir_handle* h : b->passes) freeProfile(h);
+            continue;
+        }
+        if (mixed) return bfail(b, VRESTIR_EUNSUPPORTED, "passes differ in the form of their temporal reuse");
+        break;
     }
     // temporal reuse on the previous frame's grids (an animated volume) runs as one kernel
     if (temporalTK == 0) {
@@ -2331,6 +2444,8 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
         for (int i = 0; i < n && b->ops[k] >= 0; i++) {
             const LaunchArgs& a = b->argsHost[(size_t)k * kMaxBatch + i];
             const vrestir_handle* h = b->passes[i];
+            if (a.frame.prof.tau && a.frame.prof.tau != (float*)h->profTau.p)
+                return bfail(b, VRESTIR_ESTATE, "profile rows changed while the frame was built");
             if (a.splitTK && (a.split.recs != h->split.recs || a.split.trs != h->split.trs ||
                               a.split.dens != h->split.dens || a.split.counts != h->split.counts))
                 return bfail(b, VRESTIR_ESTATE, "record buffers changed while the frame was built");
