@@ -501,8 +501,8 @@ int32_t vrestir_grid_info(const vrestir_handle* h, int32_t slot, int32_t dims[3]
 /* ---- batches: many passes in one persistent launch per step (no counterpart in the
  * reference, which renders one view per pass). Each step of a frame -- a stage, or
  * one record / trace / replay pass of a split stage -- runs as ONE persistent
- * launch whose workgroups take 16x16-pixel tiles (256-pixel ranges for the
- * traces) of every pass from a work queue in device memory; the frame's launches
+ * launch whose workgroups take 16x16-pixel tiles (ranges of at most 128 pixels for
+ * the traces) of every pass from a work queue in device memory; the frame's launches
  * are captured into a HIP graph and replayed. The passes keep their own volumes,
  * lights, cameras, resolutions and histories, and give the same images as when
  * rendered one by one; they must share path length and spatial rounds and run

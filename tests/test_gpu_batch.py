@@ -115,6 +115,18 @@ def test_batch_with_emissive_triangles_matches_passes_rendered_alone():
     compare(singles(specs), batched(specs, tuning=(64, 2, True)), specs)
 
 
+def test_batch_of_passes_with_different_marches_matches_passes_rendered_alone():
+    """Passes whose rays walk one grid with one filter beside passes whose lighting rays
+    take another mip or filter and a pass whose volume is empty: each takes the march it
+    takes alone."""
+    specs = batch_specs()
+    specs[1].params.update(spatialLightingMipLevel=0)
+    specs[2].params.update(spatialLightingUseLinearSampler=0)
+    specs[3].density = np.zeros_like(specs[3].density)
+    say("case: batch of 5 passes: default, other lighting mip, other lighting filter, empty volume, default")
+    compare(singles(specs), batched(specs, tuning=(64, 2, True)), specs)
+
+
 def test_batch_after_autotune_matches_passes_rendered_alone():
     specs = batch_specs()
     say("case: autotuned batch, then 3 frames from a reset history")

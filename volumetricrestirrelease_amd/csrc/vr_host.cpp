@@ -2302,11 +2302,15 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
     steps.push_back({learned ? kOpTraceLearned : kOpTrace, VRESTIR_STAGE_TRACE_RAYS, 0});
     if (learned) steps.push_back({-2, VRESTIR_STAGE_LEARNED_TRAIN, 0});
     steps.push_back({kOpTemporalRecord, VRESTIR_STAGE_TEMPORAL_REUSE, 0});
+    // each pass takes the march that it takes alone (LaunchArgs::traceFlat); a step that no
+    // pass takes is not launched
+    steps.push_back({kOpMarchFlat, VRESTIR_STAGE_TEMPORAL_REUSE, 0});
     steps.push_back({kOpSegmentsMarch, VRESTIR_STAGE_TEMPORAL_REUSE, 0});
     steps.push_back({kOpTemporalReplay, VRESTIR_STAGE_TEMPORAL_REUSE, 0});
     steps.push_back({kOpCopyFeatures, VRESTIR_STAGE_TEMPORAL_REUSE, 0});
     for (int r = 0; r < p0.spatialReuseRounds; r++) {
         steps.push_back({kOpSpatialRecord, VRESTIR_STAGE_SPATIAL_REUSE, r});
+        steps.push_back({kOpMarchFlat, VRESTIR_STAGE_SPATIAL_REUSE, r});
         steps.push_back({kOpSegmentsMarch, VRESTIR_STAGE_SPATIAL_REUSE, r});
         steps.push_back({kOpSpatialReplay, VRESTIR_STAGE_SPATIAL_REUSE, r});
     }
@@ -2354,7 +2358,7 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
         }
         for (size_t k = 0; k < steps.size() && rc == VRESTIR_OK; k++) {
             const Step& sp = steps[k];
-            if (sp.op < 0) continue;
+            if (sp.op < 0 || sp.op == kOpMarchFlat) continue;
             for (int i = 0; i < n && rc == VRESTIR_OK; i++) {
                 vrestir_handle* h = b->passes[i];
                 LaunchArgs tmp;
@@ -2388,24 +2392,24 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
         for (const Step& sp : steps) {
             if (sp.op == kOpTemporalRecord) s2.push_back({kOpTemporalDirect, VRESTIR_STAGE_TEMPORAL_REUSE, 0});
             else if (!(sp.stage == VRESTIR_STAGE_TEMPORAL_REUSE &&
-                       (sp.op == kOpSegmentsMarch || sp.op == kOpTemporalReplay)))
+                       (sp.op == kOpSegmentsMarch || sp.op == kOpMarchFlat || sp.op == kOpTemporalReplay)))
                 s2.push_back(sp);
         }
         steps.swap(s2);
         S = (int)steps.size();
     }
-    b->ops.assign(S, 0);
-    b->occ.assign(S, 0);
-    std::vector<int> key = {n, S, b->grid, b->per};
-    for (int k = 0; k < S; k++) {
-        const Step& sp = steps[k];
+    b->ops.clear();
+    b->occ.clear();
+    std::vector<int> key = {n, b->grid, b->per};
+    for (const Step& sp : steps) {
+        const int k = (int)b->ops.size();
         BatchList& L = b->listsHost[k];
         std::memset(&L, 0, sizeof(L));
         L.n = n;
         L.per = b->per;
-        b->ops[k] = sp.op;
-        if (sp.op < 0) { key.push_back(sp.op); continue; }
-        for (int i = 0; i < n; i++) {
+        int occ = 0;
+        std::vector<int> shape;
+        for (int i = 0; i < n && sp.op >= 0; i++) {
             vrestir_handle* h = b->passes[i];
             LaunchArgs& a = b->argsHost[(size_t)k * kMaxBatch + i];
             int rc = stageArgs(h, b->stream, sp.stage, sp.round,
@@ -2421,24 +2425,29 @@ static int batchFrame(vrestir_batch* b, hipStream_t user, const int32_t* widths,
             if (needSplit && (a.splitTK != wantTK || a.splitMode != 2))
                 return bfail(b, VRESTIR_EUNSUPPORTED, std::string("pass ") + std::to_string(i) +
                                                          ": a stage of this pass does not run in its split form");
-            if (sp.op == kOpSegmentsMarch && i == 0) b->ops[k] = kOpMarchFlat;
-            if (sp.op == kOpSegmentsMarch && !a.traceFlat) b->ops[k] = kOpSegmentsMarch;
-            const bool seg = sp.op == kOpSegmentsMarch || sp.op == kOpSegmentsCells;
+            const bool seg = sp.op == kOpSegmentsMarch || sp.op == kOpMarchFlat || sp.op == kOpSegmentsCells;
+            const bool takes = sp.op == kOpMarchFlat ? a.traceFlat != 0 : sp.op == kOpSegmentsMarch ? a.traceFlat == 0
+                               : sp.op == kOpProfile ? a.frame.prof.tau != nullptr : true;
             const int W = a.width, H = a.height;
             const int per = 4 * (64 >> a.frame.traceShift);  // pixels a workgroup of a trace
             const int gx = seg ? (W * H + per - 1) / per : (W + 15) / 16;
-            const int tiles = seg ? gx : gx * ((H + 15) / 16);
+            const int tiles = !takes ? 0 : seg ? gx : gx * ((H + 15) / 16);
             L.gx[i] = gx;
             L.tiles[i] = tiles;
             L.start[i + 1] = L.start[i] + (tiles + L.per - 1) / L.per;
-            b->occ[k] = std::max(b->occ[k], a.occBytes);
-            key.push_back(a.occBytes);
-            key.push_back(tiles);
+            if (tiles > 0) occ = std::max(occ, a.occBytes);
+            shape.push_back(a.occBytes);
+            shape.push_back(tiles);
         }
-        key.push_back(b->ops[k]);
+        if (sp.op >= 0 && L.start[n] == 0) continue;  // no pass takes the step: the next one has its place
+        b->ops.push_back(sp.op);
+        b->occ.push_back(occ);
+        key.push_back(sp.op);
+        key.insert(key.end(), shape.begin(), shape.end());
         if (sp.stage == VRESTIR_STAGE_SPATIAL_REUSE && sp.op == kOpSpatialReplay)
             for (int i = 0; i < n; i++) b->passes[i]->totalRoundId++;
     }
+    S = (int)b->ops.size();
     // every staged record buffer must be the one its pass holds now
     for (int k = 0; k < S; k++)
         for (int i = 0; i < n && b->ops[k] >= 0; i++) {

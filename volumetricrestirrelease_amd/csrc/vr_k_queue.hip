@@ -882,8 +882,9 @@ hipError_t launchTraceSegments(const LaunchArgs& a, const Options& opt, bool isF
     return hipGetLastError();
 }
 
-// The segment traces of a batched step: work items are 256-pixel ranges of one
-// instance (its recorded rays), the same ranges a plain launch gives a workgroup.
+// The segment traces of a batched step: work items are ranges of one instance's pixels
+// (its recorded rays), the ranges of 4 (64 >> traceShift) pixels that a plain launch gives
+// a workgroup. A pass that kTraceMarch takes has no tiles in this step.
 // Held to the plain kernel's four waves per SIMD: left to itself the compiler
 // gives the persistent loop 175 VGPRs (two waves), and the trace, latency bound,
 // runs about a quarter slower.
@@ -914,7 +915,7 @@ VR_TRACING_KERNEL void kBatchedSegments(const LaunchArgs* __restrict__ args,
     }
 }
 
-// kTraceMarch over a batch's items (every instance's step is flat)
+// kTraceMarch over the items of a batch's flat passes (the others have no tiles)
 VR_TRACING_KERNEL void kBatchedMarch(const LaunchArgs* __restrict__ args, const BatchList* __restrict__ list,
                                      int* __restrict__ counter) {
     __shared__ MarchShared sh;
