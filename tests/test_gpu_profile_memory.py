@@ -144,3 +144,26 @@ def test_rows_are_given_back():
     g.execute(small)
     assert free_bytes() - c > 2.6 * GB
     assert lib.vrestir_set_tuning(g.h, abi.TUNE_PROFILE_MB, -1) == abi.VRESTIR_EINVAL
+
+
+@pytest.mark.parametrize("height,rounds,rows", [(767, 0, True), (769, 0, False), (769, 1, True)])
+def test_rows_where_they_are_worth_their_making(height, rounds, rows):
+    """Without spatial rounds only frames of at most 786,432 pixels make rows (0.6 GB at
+    these sizes, about 200 march steps)."""
+    import torch
+    say(f"case: 1024x{height}, {rounds} spatial rounds: rows {rows}")
+    spec = small_scene(width=1024, height=height, maxBounces=1, initialM=1, spatialReuseRounds=1, spatialSampleCount=2,
+                       enableSpatialReuse=rounds, spatialVisibilityTStepScale=0.25)
+    out = torch.zeros((height, 1024, 4), device="cuda")
+    taken = []
+    for budget in (16384, 0):
+        g = VolumetricReSTIR()
+        g.setScene(spec)
+        assert abi.load_library().vrestir_set_tuning(g.h, abi.TUNE_PROFILE_MB, budget) == 0
+        a = free_bytes()
+        g.execute(out)
+        taken.append(a - free_bytes())
+        g.close()
+    diff = taken[0] - taken[1]
+    say(f"   {diff / GB:.2f} GB")
+    assert (0.5 * GB < diff < 0.9 * GB) if rows else abs(diff) < 0.1 * GB

@@ -1402,14 +1402,25 @@ extern "C" int32_t vrestir_learned_train(vrestir_handle* h, void* stream, const 
     return learnedStep(h, (hipStream_t)stream, recsDev, n);
 }
 
-// Whether the open frame's options use camera-ray profiles: the spatial rays are
-// ray-marched and the stages run in their split forms (the kernels of other tracker
-// mixes trace every ray and would not read them).
+// Whether the open frame uses camera-ray profiles: its options ray-march the spatial rays
+// and run the stages in their split forms (the kernels of other tracker mixes trace every
+// ray and would not read them), and the rows are worth their making. With a spatial round
+// they are at every size measured. Without one a pixel's row serves TraceRays' and at most
+// one of temporal reuse's evaluations: a small frame still gains, as the march rides along
+// in a launch that leaves the chip idle; a large one pays for the rows' writing. Frame in
+// us, with / without rows, no spatial rounds, path length 2, 128^3 and 512^3: 800x450
+// 1299 / 1321 and 3350 / 3470, 1100x620 1612 / 1607 and 3842 / 3903, 1280x720 1880 / 1849 and
+// 4249 / 4263, 1440x810 2172 / 2106 and 4642 / 4615; 1080p, path length 3 at 512^3
+// 10890 / 10710, path length 1 4770 / 4565. With one round of two neighbours there
+// 11210 / 11150 and 5232 / 5248, of three at path length 1 5585 / 6040.
+static const int kProfilePixelsAlone = 3 << 18;
 static bool profileWanted(const vrestir_handle* h) {
     const Frame& F = h->frame;
     const Options& so = F.spatialOpt;
-    return h->splitReuse == 2 && h->profBudget > 0 && so.visibilityTrackingMethod == 2u &&
-           so.lightingTrackingMethod == 2u && !F.useReference && !F.useSurfaceScene && !F.noReuse && !h->freezeFrame;
+    if (h->splitReuse != 2 || h->profBudget == 0 || so.visibilityTrackingMethod != 2u || so.lightingTrackingMethod != 2u ||
+        F.useReference || F.useSurfaceScene || F.noReuse || h->freezeFrame)
+        return false;
+    return (F.enableSpatial && F.spatialRounds > 0) || F.width * F.height <= kProfilePixelsAlone;
 }
 
 // Frame set-up: reallocation, history reset on option change, round
