@@ -111,6 +111,7 @@ struct vrestir_handle {
     DevBuf profTau, profMeta;
     bool profReady = false;
     hipStream_t profStream = nullptr;
+    unsigned long long profCapture = 0;  // the stream capture they were recorded in (0: none, they ran)
     size_t profBudget = kProfileBudget;  // VRESTIR_TUNE_PROFILE_MB
     size_t profRefused = 0;              // bytes the device had no room for (until options or size change)
     bool reserving = false;              // a batch's reservation pass: records only, no profiles
@@ -1893,6 +1894,17 @@ static int stageArgs(vrestir_handle* h, hipStream_t st, int stage, int round, fl
     return VRESTIR_OK;
 }
 
+// The capture that records stream st, 0 when none does.
+static unsigned long long captureId(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(st, &status, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusActive ? id : 0;
+}
+
 extern "C" int32_t vrestir_run_stage(vrestir_handle* h, void* stream, int32_t stage, int32_t round, float* outRGBA) {
     if (!h) return VRESTIR_EINVAL;
     if (!h->frameOpen) return fail(h, VRESTIR_ESTATE, "vrestir_prepare_frame must precede stages");
@@ -1908,11 +1920,16 @@ extern "C" int32_t vrestir_run_stage(vrestir_handle* h, void* stream, int32_t st
     const size_t n = (size_t)h->W * h->H, ne = n * (size_t)std::max(p.maxBounces - 1, 1);
     const int t = h->totalRoundId;
     // the profiles: GenerateFeatures makes them; a stage run without it, or on another
-    // stream than they were made on, makes its own first
+    // stream or in another capture than they were made in, makes its own first. (A graph
+    // captured from a later stage on is replayed after other frames' rows have taken the
+    // buffers, and rows made in a capture are not there until its graph runs.)
     if (a.frame.prof.tau) {
-        if (stage != VRESTIR_STAGE_GENERATE_FEATURES && (!h->profReady || h->profStream != st)) HIPCHK(h, launchProfile(a));
+        const unsigned long long capture = captureId(st);
+        const bool made = h->profReady && h->profStream == st && h->profCapture == capture;
+        if (stage != VRESTIR_STAGE_GENERATE_FEATURES && !made) HIPCHK(h, launchProfile(a));
         h->profReady = true;
         h->profStream = st;
+        h->profCapture = capture;
     }
     HIPCHK(h, launchStage(a));
     if (stage == VRESTIR_STAGE_TEMPORAL_REUSE) {
