@@ -317,7 +317,18 @@ enum {
     VRESTIR_BUF_TRACE_REDONE = 11,
     /* surface scenes: the V-buffer of GenerateFeatures, per pixel {int32 triangle (-1: no
      * hit), float barycentric weights of vertices 1 and 2, float ray distance (FLT_MAX)} */
-    VRESTIR_BUF_VBUFFER = 12
+    VRESTIR_BUF_VBUFFER = 12,
+    /* the last stage that ran in its split form: int32 rays per pixel; the rays, per pixel
+     * the stage's slots of {float origin[3], tMax, direction[3]; int32 kind (0: traced with
+     * the visibility options, 1: the lighting options)}; their transmittances, float
+     * [slot][pixel] */
+    VRESTIR_BUF_RAY_COUNTS = 13,
+    VRESTIR_BUF_RAYS = 14,
+    VRESTIR_BUF_RAY_TRANSMITTANCES = 15,
+    /* + grid slot: 4096 bytes, per group of (1 << s)^3 brick cells (the smallest s with at
+     * most 16 groups a side; x fastest) a bit per ray octant (bit 0 of the octant: x does
+     * not decrease, 1: y, 2: z): an occupied brick lies in the group or ahead of it */
+    VRESTIR_BUF_AHEAD = 64
 };
 int32_t vrestir_prepare_frame(vrestir_handle* h, int32_t width, int32_t height);
 int32_t vrestir_run_stage(vrestir_handle* h, void* stream, int32_t stage, int32_t round, float* outRGBA);

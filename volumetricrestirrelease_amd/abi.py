@@ -39,7 +39,8 @@ STAGE_GENERATE_FEATURES, STAGE_TRACE_RAYS, STAGE_TEMPORAL_REUSE, STAGE_SPATIAL_R
 STAGE_LEARNED_PROPOSAL, STAGE_LEARNED_TRAIN = 6, 7
 BUF_FEATURES, BUF_TEMPORAL_FEATURES, BUF_RESERVOIRS0, BUF_RESERVOIRS1, BUF_TEMPORAL_RESERVOIRS, \
     BUF_EXTRA0, BUF_EXTRA1, BUF_TEMPORAL_EXTRA, BUF_COLOR, BUF_LEARNED_CDF, BUF_TRAIN_RECORDS, \
-    BUF_TRACE_REDONE, BUF_VBUFFER = range(13)
+    BUF_TRACE_REDONE, BUF_VBUFFER, BUF_RAY_COUNTS, BUF_RAYS, BUF_RAY_TRANSMITTANCES = range(16)
+BUF_AHEAD = 64  # + grid slot
 
 TRACK_TR_ANALYTIC, TRACK_TR_RAY_MARCHING, TRACK_TR_RATIO, TRACK_TR_RESIDUAL_RATIO, \
     TRACK_TR_ANALOG_RESIDUAL_RATIO, TRACK_SAMPLE_ANALYTIC, TRACK_SAMPLE_DECOMPOSITION, \

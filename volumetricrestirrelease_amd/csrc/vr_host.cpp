@@ -107,6 +107,7 @@ struct vrestir_handle {
     bool inBatch = false;  // staged by a batch, whose TraceRays step is one kernel
     SplitBufs split{};
     size_t splitPixels = 0;
+    int splitUsed = 0;  // slots per pixel of the last stage run in its split form
     // the open frame's camera-ray profiles: the buffers, and whether they are made (on which stream)
     DevBuf profTau, profMeta;
     bool profReady = false;
@@ -196,6 +197,7 @@ static void freeSplit(vrestir_handle* h) {
     dfree(h->split.fix);
     h->split.cap = 0;
     h->splitPixels = 0;
+    h->splitUsed = 0;
 }
 static void freeFrameBuffers(vrestir_handle* h) {
     freeSplit(h);
@@ -1932,6 +1934,7 @@ extern "C" int32_t vrestir_run_stage(vrestir_handle* h, void* stream, int32_t st
         h->profCapture = capture;
     }
     HIPCHK(h, launchStage(a));
+    if (a.splitTK) h->splitUsed = a.split.cap;
     if (stage == VRESTIR_STAGE_TEMPORAL_REUSE) {
         if (!p.enableSpatialReuse) {
             HIPCHK(h, hipMemcpyAsync(h->resT, h->res[t % 2], n * sizeof(ResStore), hipMemcpyDeviceToDevice, st));
@@ -2005,6 +2008,11 @@ static int bufInfo(vrestir_handle* h, int id, void** dev, size_t& elems, int& ki
     int B = h->allocB;
     size_t ne = n * (size_t)(B > 1 ? B - 1 : 0);
     kind = 0;
+    if (id >= VRESTIR_BUF_AHEAD && id < VRESTIR_BUF_AHEAD + kMaxSlots) {
+        *dev = const_cast<uint8_t*>(h->sceneHost.grid[id - VRESTIR_BUF_AHEAD].ahead);
+        elems = kAheadBytes;
+        return 0;
+    }
     switch (id) {
         case VRESTIR_BUF_FEATURES: *dev = h->features; elems = n * 8; return 0;
         case VRESTIR_BUF_TEMPORAL_FEATURES: *dev = h->featuresT; elems = n * 8; return 0;
@@ -2018,6 +2026,12 @@ static int bufInfo(vrestir_handle* h, int id, void** dev, size_t& elems, int& ki
         case VRESTIR_BUF_LEARNED_CDF: *dev = h->lCdf; elems = h->lCdfPixels * 64; return 0;
         case VRESTIR_BUF_TRAIN_RECORDS: *dev = h->lRecs; elems = (size_t)h->lRecSlots * kLearnedRecFloats * 4; return 0;
         case VRESTIR_BUF_TRACE_REDONE: *dev = h->split.fix; elems = 4; return 0;
+        case VRESTIR_BUF_RAY_COUNTS: *dev = h->split.counts; elems = n * 4; return 0;
+        case VRESTIR_BUF_RAYS: *dev = h->split.recs; elems = n * (size_t)h->splitUsed * sizeof(TraceRec); return 0;
+        case VRESTIR_BUF_RAY_TRANSMITTANCES:
+            *dev = h->split.trs;
+            elems = n * (size_t)h->splitUsed * sizeof(float);
+            return 0;
         case VRESTIR_BUF_VBUFFER: *dev = h->vbuf; elems = n * sizeof(VItem); return 0;
     }
     return -1;

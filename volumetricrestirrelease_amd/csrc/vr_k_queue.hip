@@ -693,7 +693,9 @@ VR_DEV void marchBalanced(const Grid& Gu, MarchQueue& Q, int nSeg) {
         rem = (ow >> 8) - skip;
         brick = Q.brick[e];
         dq = V3(Q.dq[0][owner], Q.dq[1][owner], Q.dq[2][owner]);
-        q = V3(Q.q[0][e], Q.q[1][e], Q.q[2][e]) + (float)skip * dq;
+        q = V3(Q.q[0][e], Q.q[1][e], Q.q[2][e]);
+        // (the loop's positions: with the nearest filter a product's rounding changes the voxel)
+        for (int k = 0; k < skip; k++) q = q + dq;
         e++;
     };
     if (left > 0) take(f >> 8);
