@@ -28,16 +28,66 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("name", list(CASES))
-def test_profiled_camera_rays_match_marched_ones(name):
-    import torch
+def scene(name):
     c = dict(CASES[name])
-    say(f"case: camera-ray profiles against marched camera rays, {name}: {c}")
     pos, fov = c.pop("posW", None), c.pop("fovY", None)
     spec = small_scene(**{**dict(width=64, height=48, initialM=4, spatialReuseRounds=2, spatialSampleCount=4), **c})
     if pos:
         spec.camera.update(posW=pos, fovY=fov)
     spec.orbit_degrees_per_frame = 2.0
+    return spec
+
+
+def passes(spec):
+    """The pass without rows and with them: the budget is the only difference."""
+    out = []
+    for budget in (0, 16384):
+        g = VolumetricReSTIR()
+        g.setScene(spec)
+        assert abi.load_library().vrestir_set_tuning(g.h, abi.TUNE_PROFILE_MB, budget) == 0
+        out.append(g)
+    return out
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_looked_up_transmittances_are_the_marched_ones_ray_by_ray(name):
+    """TraceRays draws its sample without the rows and weighs it with the camera ray's
+    transmittance up to it: the reservoirs of every pixel hold the same sample, and p_y,
+    proportional to that transmittance, the same value (both forms add a ray's samples one
+    after the other in single precision; a few ulp where the compiler fuses differently)."""
+    import torch
+    from volumetricrestirrelease_amd.volumetric_restir import RESERVOIR_DTYPE
+    say(f"case: TraceRays' reservoirs with and without rows, {name}")
+    spec = scene(name)
+    n = spec.width * spec.height
+    both = passes(spec)
+    rays = 0
+    for f in range(4):
+        got = []
+        for g in both:
+            g.resetHistory()
+            g.setCamera(spec, f)
+            g.prepare_frame(spec.width, spec.height)
+            g.run_stage(abi.STAGE_GENERATE_FEATURES)
+            g.run_stage(abi.STAGE_TRACE_RAYS)
+            torch.cuda.synchronize()
+            got.append(g.read(abi.BUF_RESERVOIRS0, 36 * n).view(RESERVOIR_DTYPE))
+            g.end_frame()
+        a, b = got
+        for k in ("M", "depth", "lightID", "sampledPixel"):
+            assert np.array_equal(a[k], b[k]), (f, k)
+        for k in ("p_y", "runningSum"):
+            assert rel(a[k], b[k]).max() <= 2e-6, (f, k, rel(a[k], b[k]).max())
+        rays += int((a["p_y"] > 0).sum())
+    say(f"   {rays} pixels with a sample")
+    assert rays > n // 8
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_profiled_camera_rays_match_marched_ones(name):
+    import torch
+    say(f"case: camera-ray profiles against marched camera rays, {name}: {CASES[name]}")
+    spec = scene(name)
     frames = []
     for split in (0, 2):
         g = VolumetricReSTIR()

@@ -234,6 +234,9 @@ def test_device_build_at_tile_edges_equals_host_build(dims, mips, fp16, offset):
     b.setSceneStreamed(spec, buf[offset: offset + d.size])
     slots = list(range(mips)) + [8 + k for k in range(mips)]
     same_grids(a, b, slots, rng, n=4096)
+    for slot in slots:
+        ta, tb = (g.read(abi.BUF_AHEAD + slot, 4096) for g in (a, b))
+        assert np.array_equal(ta, tb), slot
     rays = np.zeros((4096, 8), np.float32)
     rays[:, :3] = rng.uniform(-1.5, 1.5, size=(4096, 3))
     dirs = rng.normal(size=(4096, 3))
@@ -243,3 +246,63 @@ def test_device_build_at_tile_edges_equals_host_build(dims, mips, fp16, offset):
         ta = track(a, abi.TRACK_TR_RESIDUAL_RATIO, slot, 1, rays)
         tb = track(b, abi.TRACK_TR_RESIDUAL_RATIO, slot, 1, rays)
         assert np.array_equal(ta.view(np.uint32), tb.view(np.uint32)), slot
+
+
+def ahead_table(occ):
+    """VRESTIR_BUF_AHEAD from brick occupancy [z, y, x]: groups of the smallest power of
+    two cells that leave at most 16 a side, then per octant a running OR from the far end."""
+    s = 0
+    while max(((n - 1) >> s) + 1 for n in occ.shape) > 16:
+        s += 1
+    g = 1 << s
+    shape = [((n - 1) >> s) + 1 for n in occ.shape]
+    pad = np.zeros([n * g for n in shape], bool)
+    pad[: occ.shape[0], : occ.shape[1], : occ.shape[2]] = occ
+    groups = pad.reshape(shape[0], g, shape[1], g, shape[2], g).any(axis=(1, 3, 5))
+    out = np.zeros(shape, np.uint8)
+    for o in range(8):
+        v = groups
+        for axis, up in ((2, o & 1), (1, (o >> 1) & 1), (0, o >> 2)):
+            v = np.logical_or.accumulate(np.flip(v, axis), axis) if up else np.logical_or.accumulate(v, axis)
+            v = np.flip(v, axis) if up else v
+        out |= v.astype(np.uint8) << o
+    flat = np.zeros(4096, np.uint8)
+    flat[: out.size] = out.reshape(-1)
+    return flat, s
+
+
+@pytest.mark.parametrize("dims,where", [((64, 64, 64), "one"), ((136, 128, 40), "few"), ((264, 136, 520), "few"),
+                                        ((1032, 264, 1024), "few"), ((128, 128, 128), "none"),
+                                        ((2056, 128, 128), "corners")])
+def test_ahead_table_is_the_occupancys(dims, where):
+    """The table that ends walks, of the GPU build and of the host build, from grids of few
+    bricks: sides on both sides of 16 groups (shifts 0 to 5), slots on both sides of the
+    one-workgroup table pass, no brick at all."""
+    import torch
+    nx, ny, nz = dims
+    say(f"case: {nx}x{ny}x{nz}, bricks: {where}")
+    rng = np.random.default_rng(nx + ny)
+    d = np.zeros((nz, ny, nx), np.float32)
+    if where == "corners":
+        d[0, 0, 0] = d[-1, -1, -1] = d[0, -1, nx // 2] = 1.0
+    elif where != "none":
+        for _ in range(1 if where == "one" else 9):
+            d[rng.integers(nz), rng.integers(ny), rng.integers(nx)] = 0.5
+    occ = d.reshape(nz // 8, 8, ny // 8, 8, nx // 8, 8).max(axis=(1, 3, 5)) > 0
+    spec = small_scene(res=8, width=16, height=8)
+    spec.density, spec.num_mips = d, 1
+    m = np.zeros(16, np.float32)
+    m[0], m[5], m[10], m[15] = 2.0 / nx, 2.0 / ny, 2.0 / nz, 1.0
+    m[12:15] = -1.0
+    spec.index_to_world = m
+    spec.params.update(initialBaseMipLevel=0, initialLightingMipLevel=0, temporalReprojectionMipLevel=0,
+                       spatialVisibilityMipLevel=0, spatialLightingMipLevel=0)
+    want, shift = ahead_table(occ)
+    say(f"   shift {shift}, {int(occ.sum())} bricks of {occ.size}")
+    a = VolumetricReSTIR()
+    a.setScene(spec)
+    b = VolumetricReSTIR()
+    b.setSceneStreamed(spec, dev(d))
+    torch.cuda.synchronize()
+    assert np.array_equal(a.read(abi.BUF_AHEAD, 4096), want)
+    assert np.array_equal(b.read(abi.BUF_AHEAD, 4096), want)
