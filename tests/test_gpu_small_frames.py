@@ -1,13 +1,15 @@
 """Frames of every size class of the launch spread: small frames give each wave a few
 pixels (down to four in the stage kernels, one in the segment traces), larger ones 64.
-The spread changes which wave a pixel is in and nothing else, so the top-left region of
-the first frame, which depends on the pixel alone, is the oracle's for every size."""
+The spread changes which wave a pixel is in and nothing else: a frame equals, bit for bit
+and in every row and column, the one that a batch of one pass renders with 64 pixels a
+wave, and its middle rows, whose neighbours the oracle has traced too, are the oracle's."""
 import numpy as np
 import pytest
 
 from gpu_common import say, small_scene
 from oracle.binding import Oracle
-from volumetricrestirrelease_amd.volumetric_restir import VolumetricReSTIR
+from volumetricrestirrelease_amd import abi
+from volumetricrestirrelease_amd.volumetric_restir import VolumetricReSTIR, VolumetricReSTIRBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +41,35 @@ def test_frame_of_any_spread_matches_the_oracle(width, height):
     say(f"   pixels within 1e-3: {frac:.4f}")
     # the bar of whole uninjected frames (comparisons that rounding flips on single pixels)
     assert frac >= 0.97
+
+
+@pytest.mark.parametrize("width,height", [(1, 1), (1, 200), (17, 3), (37, 1), (64, 63), (100, 61), (129, 127), (255, 257),
+                                          (390, 333), (513, 509), (600, 450)])
+def test_frame_of_any_spread_equals_the_unspread_one(width, height):
+    """Widths and heights that leave remainders of the 16-wide tiles and of their 16, 8, 4, 2
+    and 1 rows; the images start as NaN. (A batch runs TraceRays in one kernel: so does the
+    pass alone here.)"""
+    import torch
+    say(f"case: {width}x{height} frame alone against a batch of one")
+    spec = small_scene(res=32, width=width, height=height, maxBounces=3, initialM=3, spatialReuseRounds=1,
+                       spatialSampleCount=3)
+    imgs = []
+    for batch in (False, True):
+        g = VolumetricReSTIR()
+        g.setScene(spec)
+        assert abi.load_library().vrestir_set_tuning(g.h, abi.TUNE_SPLIT_TRACE, 0) == 0
+        out = torch.full((height, width, 4), float("nan"), device="cuda")
+        if batch:
+            b = VolumetricReSTIRBatch([g])
+            b.execute([out])
+        else:
+            g.execute(out)
+        torch.cuda.synchronize()
+        imgs.append(out.cpu().numpy())
+        if batch:
+            b.close()
+    assert np.isfinite(imgs[0]).all() and np.isfinite(imgs[1]).all()
+    assert np.array_equal(imgs[0], imgs[1])
 
 
 @pytest.mark.parametrize("points", [1, 7, 700, 5000])

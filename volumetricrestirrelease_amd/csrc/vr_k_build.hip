@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kBuildThreads) void kClear(unsigned* __restrict__ p
 // level by level, and each level's values and bricks' largest values written. A tile
 // without a positive value (most of a sparse volume) writes its zeros and ends.
 // Tiles wider in x than the 128-byte lines they touch, 8 deep so that level 3 and the
-// bricks need no exchange between workgroups; 47 KB of LDS, three workgroups per CU.
+// bricks need no exchange between workgroups; 50 KB of LDS, three workgroups per CU.
 constexpr int kTX = 64, kTY = 8, kTZ = 8;
 constexpr int kRow = 72;  // LDS row: voxel x at 4 + x, so that 16-byte stores align
 struct LevelGrids {
