@@ -35,23 +35,25 @@ VR_SEG_FN int segmentLoop(float t, float qx, float qy, float qz, float dx, float
 // forming the samples here costs as much again: the margins are these sums, rounded up.
 // Positions move one way on each axis, so the samples between the first and the last are
 // inside too. Everything else (rays that graze a face, times within rounding of tFar, 128
-// samples, NaN) gives -1: the loop tells. Where the guess comes from does not matter for the result:
-// the walk's exit time carries the rounding of grid coordinates divided by the direction,
-// up to several steps for rays that graze a face, so a bound on the time alone will not do.
+// samples, NaN) gives -1 and the loop tells: 2e-4 to 3e-3 of the segments with a sample at
+// 0.2 to 2 voxels a step. Where the guess comes from does not matter for the result: the
+// walk's exit time carries the rounding of grid coordinates divided by the direction, up to
+// several steps for rays that graze a face, so a bound on the time alone will not do.
 VR_SEG_FN int segmentCertain(float r, float t0, float qx, float qy, float qz, float dx, float dy, float dz,
                              float tStep, float tFar) {
+    const bool first = qx >= 0.f && qy >= 0.f && qz >= 0.f && qx < 8.f && qy < 8.f && qz < 8.f;
+    if (!(first && t0 < tFar)) return 0;
     const float nf = ceilf(r);
     if (!(nf >= 1.f && nf < 128.f)) return -1;
     const float k = nf - 1.f, m = 3e-7f * (nf + 3.f);
     const float tm = 8e-8f * (nf + 1.f) * (fabsf(t0) + nf * tStep);
-    const bool first = qx >= 0.f && qy >= 0.f && qz >= 0.f && qx < 8.f && qy < 8.f && qz < 8.f;
     const float lx = fmaf(k, dx, qx), ly = fmaf(k, dy, qy), lz = fmaf(k, dz, qz), tl = fmaf(k, tStep, t0);
     const float lo = fminf(fminf(lx, ly), lz), hi = fmaxf(fmaxf(lx, ly), lz);
     const bool last = lo >= m && hi < 8.f - m && tl + tm < tFar;
     const float ox = lx + dx, oy = ly + dy, oz = lz + dz, sum = ox + oy + oz;
     const float low = fminf(fminf(ox, oy), oz), high = fmaxf(fmaxf(ox, oy), oz);
     const bool past = high - 8.f > m + 2e-7f * high || -low > m - 2e-7f * low || tl + tStep - tm >= tFar;
-    return first && last && past && sum == sum ? (int)nf : -1;  // (min and max pass a NaN axis over)
+    return last && past && sum == sum ? (int)nf : -1;  // (min and max pass a NaN axis over)
 }
 VR_SEG_FN int segmentCount(float r, float t0, float qx, float qy, float qz, float dx, float dy, float dz, float tStep,
                            float tFar) {
