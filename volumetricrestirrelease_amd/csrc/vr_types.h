@@ -215,16 +215,17 @@ struct Frame {
 // runs as long as the longest of its lanes' walks, one divergent path after another, so a
 // launch too small to fill the chip many times over finishes sooner with fewer pixels a
 // wave and more waves, up to `waves` of them. Four waves of the tracing kernels reside on
-// each of 1024 SIMDs. Measured (frame, us; one wave a 64 pixels first):
-//   stage kernels: 4096 waves, 4 pixels at least: 96x64 957 -> 748 together with the
-//     traces; 2048: 480x270 +5 %, 8192: 640x360 +6 %;
+// each of 1024 SIMDs. Measured, 64 pixels a wave everywhere against the spread below:
+// 96x64 905 -> 745 us, 480x270 animated 2240 -> 1690, 640x360 1720 -> 1388, 797x451 emissive
+// 2943 -> 2737, 960x540 learned 9275 -> 8135. The limits, other values against the taken one:
+//   stage kernels: 4096 waves, 4 pixels at least (2048: 480x270 +5 %, 8192: 640x360 +6 %);
 //   segment traces (a wave keeps its 64 lanes busy from its pixels' rays, so more waves
-//     only cost their set-up): 16384, one pixel at least: 640x360 1607 -> 1280, 400x225
-//     2743 (4096 waves) -> 2150; 8192: 640x360 1361, 32768: 1337, 480x270 +3 %; and never
-//     more than 32 pixels: 1080p 28.2 -> 26.6 ms (16: 26.5), six views of 256^2 to 1440x810
-//     in a batch 24.6 -> 24.3 (with 65536 waves: 25.6);
+//     only cost their set-up): 16384, one pixel at least (4096: 400x225 +28 %; 8192:
+//     640x360 +6 %, 32768: +4 %); and never more than 32 pixels: 1080p 22.95 -> 21.11 ms
+//     (16: the same), six views of 256^2 to 1440x810 in a batch 24.13 -> 23.66 (65536 waves:
+//     +5 %);
 //   path-traced lattices (lanes that end leave the wave idle): 8192: 240x135 points x 4
-//     14.1 -> 12.3 ms; 4096: 13.4.
+//     14.56 -> 12.13 ms (4096: +9 %).
 // Sums of a ray's optical depth depend on the segment traces' spread (their order), so a
 // batch gives each of its passes the spread it has alone.
 inline int laneShiftFor(int64_t n, int64_t waves, int most) {
