@@ -318,7 +318,8 @@ enum {
     /* surface scenes: the V-buffer of GenerateFeatures, per pixel {int32 triangle (-1: no
      * hit), float barycentric weights of vertices 1 and 2, float ray distance (FLT_MAX)} */
     VRESTIR_BUF_VBUFFER = 12,
-    /* the last stage that ran in its split form: int32 rays per pixel; the rays, per pixel
+    /* read only from here on.
+     * The last stage that ran in its split form: int32 rays per pixel; the rays, per pixel
      * the stage's slots of {float origin[3], tMax, direction[3]; int32 kind (0: traced with
      * the visibility options, 1: the lighting options)}; their transmittances, float
      * [slot][pixel] */

@@ -306,3 +306,7 @@ def test_ahead_table_is_the_occupancys(dims, where):
     torch.cuda.synchronize()
     assert np.array_equal(a.read(abi.BUF_AHEAD, 4096), want)
     assert np.array_equal(b.read(abi.BUF_AHEAD, 4096), want)
+    with pytest.raises(VolumetricReSTIRError, match="read only"):
+        b.write(abi.BUF_AHEAD, want)
+    with pytest.raises(VolumetricReSTIRError, match="unallocated"):
+        b.read(abi.BUF_AHEAD + 1, 4096)  # mip 1 is not bound

@@ -2066,6 +2066,7 @@ extern "C" int32_t vrestir_read_buffer(vrestir_handle* h, int32_t id, void* dst,
 
 extern "C" int32_t vrestir_write_buffer(vrestir_handle* h, int32_t id, const void* src, size_t bytes) {
     if (!h || !src) return VRESTIR_EINVAL;
+    if (id >= VRESTIR_BUF_RAY_COUNTS) return fail(h, VRESTIR_EINVAL, "this buffer is read only");
     void* dev;
     size_t elems;
     int kind;

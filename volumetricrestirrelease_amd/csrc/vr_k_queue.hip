@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void kTraceQueue(const Scene* __restrict__ sc,
 // The same queue of recorded rays, traced in two alternating phases so that the
 // lanes of a wave run one code path at a time:
 //   * walk: every lane steps the DDA of its own ray, one cell per iteration (at
-//     brick level only when the grid's block bits fit LDS, Walker::flatSegment,
+//     brick level only when the grid's block bits fit LDS, FlatWalk,
 //     else the hierarchical walk), and pushes each occupied brick it enters (with
 //     the march's first sample) to a per-wave segment queue in LDS; a lane whose
 //     walk is over takes the next ray of the queue;

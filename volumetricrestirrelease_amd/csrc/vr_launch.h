@@ -61,7 +61,7 @@ hipError_t launchTraceCells(const LaunchArgs& a, const Options& opt, bool isFina
 // The work list of one batched step: instance i owns work items [start[i],
 // start[i+1]); an item is `per` consecutive tiles of that instance, tiles
 // row-major over its tile grid of gx columns (16x16-pixel tiles for the stage
-// bodies, 256-pixel ranges for the segment traces).
+// bodies, ranges of 4 (64 >> traceShift) pixels for the segment traces).
 constexpr int kMaxBatch = 64;
 struct BatchList {
     int n, per;
